@@ -104,11 +104,11 @@ def geometry_byte_model(nx, ny, spherical=True):
     """Algorithmic HBM bytes of one one-pass subcycle on a general mesh (CG2): per element
     the stress read and written (3 S coefficients each), the strength at the Q Gauss points
     and the geometry table (the 6 bilinear map coefficients, on the sphere cos and sin of
-    the latitude at the Q Gauss points, the upper triangle of the inverse mass matrix); per
-    node u, v read and written and the 6 frozen values read."""
+    the latitude at the Q Gauss points); per node u, v read and written and the 6 frozen
+    values read."""
     S, Q = 8, 9
     ne, nn = nx * ny, (2 * nx + 1) * (2 * ny + 1)
-    geo = 6 + (2 * Q if spherical else 0) + S * (S + 1) // 2
+    geo = 6 + (2 * Q if spherical else 0)
     return 8 * (6 * S + Q + geo) * ne + 80 * nn
 
 
@@ -166,10 +166,9 @@ def brittle_byte_model(nx, ny, cg=2, dg=6):
 
 def brittle_general_byte_model(nx, ny, cg=2, dg=6):
     """brittle_byte_model on a general (planar) mesh: plus the geometry table (6 bilinear map
-    coefficients and the upper triangle of the inverse stress mass matrix) and the brittle
-    table (h_e and the upper triangle of the inverse DG mass matrix) per element."""
-    S = 8 if cg == 2 else 3
-    return brittle_byte_model(nx, ny, cg, dg) + 8 * (6 + S * (S + 1) // 2 + 1 + dg * (dg + 1) // 2) * nx * ny
+    coefficients) and the brittle table (h_e and the upper triangle of the inverse DG mass
+    matrix) per element."""
+    return brittle_byte_model(nx, ny, cg, dg) + 8 * (6 + 1 + dg * (dg + 1) // 2) * nx * ny
 
 
 def brittle_leg(nx, steps, warmup, dt=120.0, seed=0, traffic_path=None, warp=0.0):
