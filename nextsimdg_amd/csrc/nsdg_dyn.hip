@@ -137,6 +137,43 @@ template <int CG> __global__ void k_momentum_ops(MeshView m, int nOps, double* o
     }
 }
 
+// Reciprocal, reciprocal square root, square root and quotient of the subcycle kernels: the
+// hardware's estimates (about 24 bits) refined by Newton steps to an ulp, without the range
+// scaling and special-case selects of the general functions (half their instructions; the
+// element and node updates run 9 and 4 to 8 of them per element). Arguments are normal
+// numbers away from the ends of the range: Jacobians and their weights, Delta^2 >= DeltaMin^2,
+// squared speeds, the momentum denominators.
+__device__ __forceinline__ double reciprocal(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ double quotient(double a, double b)
+{
+    const double r = reciprocal(b), q = a * r;
+    return fma(fma(-b, q, a), r, q);
+}
+// One third-order step: the estimate's error cubed is below the rounding.
+__device__ __forceinline__ double rsq(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ float rsq(float x) { return rsqrtf(x); }
+// sqrt(x) for x >= 0; below 1e-280 (speeds of 1e-140 m/s) it returns 1e-140.
+__device__ __forceinline__ double squareRoot(double x)
+{
+    x = fmax(x, 1e-280);
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    return fma(fma(-g, g, x), h, g);
+}
+
 // Per-element geometry of the one-pass subcycle on general meshes, SoA [k][ne]: the
 // bilinear map x(xi, eta) = x0 + X1 xi + X2 eta + X3 xi eta (and y), so that at any point
 // x_xi = X1 + X3 eta, x_eta = X2 + X3 xi; on the sphere cos and sin of the latitude at the
@@ -236,14 +273,6 @@ template <int CG> __device__ __forceinline__ constexpr double complementAt(int g
 }
 static_assert(GeoLayout<2>::Q == GeoLayout<2>::S + 1 && GeoLayout<1>::Q == GeoLayout<1>::S + 1,
     "the stress space leaves out one function of the Gauss tensor product");
-// 1 / x to an ulp: the hardware's estimate (24 bits) and two Newton steps; x is a normal
-// number away from the ends of the range (Jacobians, their weights and sums of them).
-__device__ __forceinline__ double reciprocal(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
-}
 // Per-element data of the brittle update on general meshes, SoA [k][ne]: the element size
 // h = sqrt(area) (ParametricMesh::area, ParametricMesh.hpp:276-299, of the stored vertices,
 // whose longitudes it does not correct), then iMJwPSI_dam (ParametricMap.cpp:290-296 and
@@ -912,8 +941,6 @@ template <class R, class C> __device__ __forceinline__ R storeValue(const Acc<C>
     else
         return roundStochastic(a, coefficientBits(elementSeed(static_cast<uint32_t>(e), it), static_cast<uint32_t>(k)));
 }
-__device__ __forceinline__ double rsq(double x) { return rsqrt(x); }
-__device__ __forceinline__ float rsq(float x) { return rsqrtf(x); }
 template <class R> __device__ __forceinline__ R* stressOf(const ElemArgs& a);
 template <> __device__ __forceinline__ double* stressOf<double>(const ElemArgs& a) { return a.sig; }
 template <> __device__ __forceinline__ float* stressOf<float>(const ElemArgs& a) { return a.sigF; }
@@ -921,12 +948,42 @@ template <class R> __device__ __forceinline__ const R* strengthOf(const ElemArgs
 template <> __device__ __forceinline__ const double* strengthOf<double>(const ElemArgs& a) { return a.Pg; }
 template <> __device__ __forceinline__ const float* strengthOf<float>(const ElemArgs& a) { return a.PgF; }
 
+// Land elements keep their stored strain: its Gauss-point values replace the velocity's in
+// a branch taken by whole waves (no divergent control flow around the element update).
+template <int CG, class C>
+__device__ __forceinline__ void landStrainGauss(const ElemArgs& a, int e, C* x11, C* x12, C* x22)
+{
+    using L = MomLayout<CG>;
+    constexpr int S = L::S, NG = L::G;
+    const uint32_t off = static_cast<uint32_t>(e) * 8u;
+    const bool land = ldAt(a.ocean, static_cast<uint32_t>(e)) == 0;
+    if (__builtin_amdgcn_ballot_w64(land) == 0)
+        return;
+    C* const x[3] = { x11, x12, x22 };
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        C s[S];
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+            s[k] = static_cast<C>(ldAt(a.eps + (c * S + k) * static_cast<size_t>(a.ne), off));
+#pragma unroll
+        for (int q = 0; q < NG * NG; ++q) {
+            double bd[8];
+            dgBasisAt(gauss_point(NG, q % NG) - 0.5, gauss_point(NG, q / NG) - 0.5, bd);
+            C g = 0;
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+                g += s[k] * static_cast<C>(bd[k]);
+            x[c][q] = land ? g : x[c][q];
+        }
+    }
+}
 // R = double: the FP64 path. R = float: strain, Delta, stress and the projection in FP32;
 // the FP64 node velocities enter relative to the element's centre node (their differences,
 // which the gradient needs, are formed exactly in FP64 before rounding to FP32).
 // VP: sigma <- Pi sigma_VP(eps(u)) outright (no relaxation, the old stress is not read);
 // used for the momentum residual and for the stress of a predicted velocity.
-// vel(lu, lv) gives the element's node velocities by node row (ocean elements only);
+// vel(lu, lv) gives the element's node velocities by node row;
 // old(c, s) the previous stress, component c (11, 12, 22), coefficient s.
 // str(q) gives the ice strength at Gauss point q (row-major, x fastest); by default it is
 // read from the strength table.
@@ -935,26 +992,67 @@ __device__ __forceinline__ void elementAffineCore(
     const ElemArgs& a, int e, Acc<C>* acc1, Acc<C>* acc2, Acc<C>* acc3, const VEL& vel, const OLD& old, const STR& str)
 {
     using L = MomLayout<CG>;
-    constexpr int S = L::S, NG = L::G, N = L::N, K = CG + 1;
-    const size_t ne = a.ne;
-    const bool oc = ldAt(a.ocean, static_cast<uint32_t>(e)) != 0;
-    C buf[3 * S]; // ocean: u (N), v (N) by node row; land: e11, e12, e22 (S each)
-    if (oc) {
-        double lu[N], lv[N];
-        vel(lu, lv);
-        const double cu = sizeof(C) == 8 ? 0.0 : lu[N / 2], cv = sizeof(C) == 8 ? 0.0 : lv[N / 2];
+    constexpr int S = L::S, NG = L::G, Q = L::Q, N = L::N, K = CG + 1;
+    // The strain at all Gauss points first, then the rheology: straight-line code, in which
+    // the loads of the strength (and of the next phase) can be issued ahead and independent
+    // points overlap. The velocity's strain is formed for land elements too (their nodes
+    // exist) and replaced afterwards.
+    C x11[Q], x12[Q], x22[Q];
+    {
+        C bu[N], bv[N];
+        {
+            double lu[N], lv[N];
+            vel(lu, lv);
+            const double cu = sizeof(C) == 8 ? 0.0 : lu[N / 2], cv = sizeof(C) == 8 ? 0.0 : lv[N / 2];
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-            buf[j] = static_cast<C>(lu[j] - cu);
-            buf[N + j] = static_cast<C>(lv[j] - cv);
+            for (int j = 0; j < N; ++j) {
+                bu[j] = static_cast<C>(lu[j] - cu);
+                bv[j] = static_cast<C>(lv[j] - cv);
+            }
         }
-    } else {
+        const C xiX = static_cast<C>(a.xiX), etaX = static_cast<C>(a.etaX);
+        const C xiY = static_cast<C>(a.xiY), etaY = static_cast<C>(a.etaY);
 #pragma unroll
-        for (int k = 0; k < 3 * S; ++k)
-            buf[k] = static_cast<C>(a.eps[k * ne + e]);
+        for (int gy = 0; gy < NG; ++gy) {
+            // velocity interpolated (Iu, Iv) and differentiated (Du, Dv) along y at this Gauss row
+            C Iu[K], Du[K], Iv[K], Dv[K];
+#pragma unroll
+            for (int jx = 0; jx < K; ++jx) {
+                C iu = 0, du = 0, iv = 0, dv = 0;
+#pragma unroll
+                for (int jy = 0; jy < K; ++jy) {
+                    const C ph = static_cast<C>(cg_1d(CG, jy, gauss_point(NG, gy)));
+                    const C dp = static_cast<C>(cg_1d_dx(CG, jy, gauss_point(NG, gy)));
+                    iu += ph * bu[jx + K * jy];
+                    du += dp * bu[jx + K * jy];
+                    iv += ph * bv[jx + K * jy];
+                    dv += dp * bv[jx + K * jy];
+                }
+                Iu[jx] = iu;
+                Du[jx] = du;
+                Iv[jx] = iv;
+                Dv[jx] = dv;
+            }
+#pragma unroll
+            for (int gx = 0; gx < NG; ++gx) {
+                C uxi = 0, ueta = 0, vxi = 0, veta = 0;
+#pragma unroll
+                for (int jx = 0; jx < K; ++jx) {
+                    const C ph = static_cast<C>(cg_1d(CG, jx, gauss_point(NG, gx)));
+                    const C dp = static_cast<C>(cg_1d_dx(CG, jx, gauss_point(NG, gx)));
+                    uxi += dp * Iu[jx];
+                    ueta += ph * Du[jx];
+                    vxi += dp * Iv[jx];
+                    veta += ph * Dv[jx];
+                }
+                const int q = gx + NG * gy;
+                x11[q] = uxi * xiX + ueta * etaX;
+                x22[q] = vxi * xiY + veta * etaY;
+                x12[q] = C(0.5) * ((uxi * xiY + ueta * etaY) + (vxi * xiX + veta * etaX));
+            }
+        }
     }
-    const C xiX = static_cast<C>(a.xiX), etaX = static_cast<C>(a.etaX);
-    const C xiY = static_cast<C>(a.xiY), etaY = static_cast<C>(a.etaY);
+    landStrainGauss<CG, C>(a, e, x11, x12, x22);
     const C DM2 = static_cast<C>(a.DM2);
     // The projected terms sum_q PSI_s(q) w_q / m_s r(q) of each coefficient, summed plainly:
     // in acc (FP64), in t (FP32).
@@ -969,78 +1067,31 @@ __device__ __forceinline__ void elementAffineCore(
         }
     }
 #pragma unroll
-    for (int gy = 0; gy < NG; ++gy) {
-        // velocity interpolated (Iu, Iv) and differentiated (Du, Dv) along y at this Gauss row
-        C Iu[K], Du[K], Iv[K], Dv[K];
-        if (oc) {
+    for (int q = 0; q < Q; ++q) {
+        double bd[8];
+        dgBasisAt(gauss_point(NG, q % NG) - 0.5, gauss_point(NG, q / NG) - 0.5, bd);
+        const C g11 = x11[q], g12 = x12[q], g22 = x22[q];
+        const C X = DM2 + C(1.25) * (g11 * g11 + g22 * g22) + C(1.50) * g11 * g22 + g12 * g12;
+        const C P = str(q);
+        const C c = (P * C(0.125)) * rsq(X); // P / (8 Delta)
+        const C w = static_cast<C>(gauss_weight(NG, q % NG) * gauss_weight(NG, q / NG)) * static_cast<C>(a.invAlpha);
+        const C r11 = w * (c * (C(5.0) * g11 + C(3.0) * g22) - C(0.5) * P);
+        const C r12 = w * ((C(2.0) * c) * g12);
+        const C r22 = w * (c * (C(5.0) * g22 + C(3.0) * g11) - C(0.5) * P);
+        // iMJwPSI[s][q] = PSI_s(q) w_q / m_s: w_q is in r, PSI_s(q) / m_s is a literal
 #pragma unroll
-            for (int jx = 0; jx < K; ++jx) {
-                C iu = 0, du = 0, iv = 0, dv = 0;
-#pragma unroll
-                for (int jy = 0; jy < K; ++jy) {
-                    const C ph = static_cast<C>(cg_1d(CG, jy, gauss_point(NG, gy)));
-                    const C dp = static_cast<C>(cg_1d_dx(CG, jy, gauss_point(NG, gy)));
-                    iu += ph * buf[jx + K * jy];
-                    du += dp * buf[jx + K * jy];
-                    iv += ph * buf[N + jx + K * jy];
-                    dv += dp * buf[N + jx + K * jy];
-                }
-                Iu[jx] = iu;
-                Du[jx] = du;
-                Iv[jx] = iv;
-                Dv[jx] = dv;
-            }
-        }
-#pragma unroll
-        for (int gx = 0; gx < NG; ++gx) {
-            double bd[8];
-            dgBasisAt(gauss_point(NG, gx) - 0.5, gauss_point(NG, gy) - 0.5, bd);
-            C g11 = 0, g12 = 0, g22 = 0;
-            if (oc) {
-                C uxi = 0, ueta = 0, vxi = 0, veta = 0;
-#pragma unroll
-                for (int jx = 0; jx < K; ++jx) {
-                    const C ph = static_cast<C>(cg_1d(CG, jx, gauss_point(NG, gx)));
-                    const C dp = static_cast<C>(cg_1d_dx(CG, jx, gauss_point(NG, gx)));
-                    uxi += dp * Iu[jx];
-                    ueta += ph * Du[jx];
-                    vxi += dp * Iv[jx];
-                    veta += ph * Dv[jx];
-                }
-                g11 = uxi * xiX + ueta * etaX;
-                g22 = vxi * xiY + veta * etaY;
-                g12 = C(0.5) * ((uxi * xiY + ueta * etaY) + (vxi * xiX + veta * etaX));
+        for (int s = 0; s < S; ++s) {
+            const double bs = bd[s] * invMassRef(s);
+            if (bs == 0.0) // basis functions vanishing at this Gauss point (a literal test)
+                continue;
+            if constexpr (sizeof(C) == 8) {
+                acc1[s].add(static_cast<C>(bs) * r11);
+                acc2[s].add(static_cast<C>(bs) * r12);
+                acc3[s].add(static_cast<C>(bs) * r22);
             } else {
-#pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    const C b = static_cast<C>(bd[s]);
-                    g11 += buf[s] * b;
-                    g12 += buf[S + s] * b;
-                    g22 += buf[2 * S + s] * b;
-                }
-            }
-            const C X = DM2 + C(1.25) * (g11 * g11 + g22 * g22) + C(1.50) * g11 * g22 + g12 * g12;
-            const C P = str(gx + NG * gy);
-            const C c = (P * C(0.125)) * rsq(X); // P / (8 Delta)
-            const C w = static_cast<C>(gauss_weight(NG, gx) * gauss_weight(NG, gy)) * static_cast<C>(a.invAlpha);
-            const C r11 = w * (c * (C(5.0) * g11 + C(3.0) * g22) - C(0.5) * P);
-            const C r12 = w * ((C(2.0) * c) * g12);
-            const C r22 = w * (c * (C(5.0) * g22 + C(3.0) * g11) - C(0.5) * P);
-            // iMJwPSI[s][q] = PSI_s(q) w_q / m_s: w_q is in r, PSI_s(q) / m_s is a literal
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const double bs = bd[s] * invMassRef(s);
-                if (bs == 0.0) // basis functions vanishing at this Gauss point (a literal test)
-                    continue;
-                if constexpr (sizeof(C) == 8) {
-                    acc1[s].add(static_cast<C>(bs) * r11);
-                    acc2[s].add(static_cast<C>(bs) * r12);
-                    acc3[s].add(static_cast<C>(bs) * r22);
-                } else {
-                    t1[s] += static_cast<C>(bs) * r11;
-                    t2[s] += static_cast<C>(bs) * r12;
-                    t3[s] += static_cast<C>(bs) * r22;
-                }
+                t1[s] += static_cast<C>(bs) * r11;
+                t2[s] += static_cast<C>(bs) * r12;
+                t3[s] += static_cast<C>(bs) * r22;
             }
         }
     }
@@ -1417,10 +1468,10 @@ __device__ __forceinline__ void momentumFrozen(const NodeArgs& a, const NodeFz& 
     double& vn)
 {
     const double uOcnRel = in.ocn.x - in.u, vOcnRel = in.v - in.ocn.y;
-    const double absocn = sqrt(uOcnRel * uOcnRel + vOcnRel * vOcnRel);
+    const double absocn = squareRoot(uOcnRel * uOcnRel + vOcnRel * vOcnRel);
     const double c1 = in.cf.x, drag = in.cf.y * absocn; // both times ML
     const double cor = c1 * a.dt * a.fc;                 // ML rho_ice H fc
-    const double inv = 1.0 / (c1 * (1.0 + a.beta) + drag);
+    const double inv = reciprocal(c1 * (1.0 + a.beta) + drag);
     un = inv * (c1 * a.beta * in.u + in.qf.x + drag * in.ocn.x - cor * in.u + dSx);
     vn = inv * (c1 * a.beta * in.v + in.qf.y + drag * in.ocn.y + cor * in.v + dSy);
 }
@@ -1443,6 +1494,42 @@ struct MevpNode {
         momentumFrozen(a, in, dx, dy, un, vn);
     }
 };
+
+// Minus the sum of a node's <= 4 contributions, in the two-colour stripe order of the
+// scatter (element rows of even index first, columns ascending): every candidate slot is
+// read and the absent ones (outside the domain; the second column or row of a node inside
+// an element) are replaced by zero, so that the four reads are in flight together instead
+// of one after the other behind a branch each. index(ex, ey) gives the local element of
+// contrib(le, j, c), its node j and component c.
+template <int CG, class I, class G>
+__device__ __forceinline__ void nodeDivergence(int nix, int niy, int nx, int ny, const I& index, const G& contrib,
+    double& dx, double& dy)
+{
+    int c[2], l[2], r[2], m[2];
+    bool hc[2], hr[2];
+    axisCandidates(CG, nix, nx, c[0], l[0], hc[0], c[1], l[1], hc[1]);
+    axisCandidates(CG, niy, ny, r[0], m[0], hr[0], r[1], m[1], hr[1]);
+    const bool swap = hr[0] && hr[1] && (r[0] & 1) != 0; // two rows, the lower of odd index
+    double x[2][2], y[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const bool has = hr[i] && hc[k];
+            const int le = has ? index(c[k], r[i]) : 0, j = has ? l[k] + (CG + 1) * m[i] : 0;
+            const double vx = static_cast<double>(contrib(le, j, 0)), vy = static_cast<double>(contrib(le, j, 1));
+            x[i][k] = has ? vx : 0.0;
+            y[i][k] = has ? vy : 0.0;
+        }
+    dx = dy = 0.0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            dx -= swap ? x[1 - i][k] : x[i][k];
+            dy -= swap ? y[1 - i][k] : y[i][k];
+        }
+}
 
 // Phase 2 of a node tile: the owned nodes sum their <= 4 contributions (contrib(le, j, c):
 // local element le, its node j, component c; two-colour stripe order, land contributions
@@ -1480,19 +1567,14 @@ __device__ __forceinline__ void nodeTileUpdate(const NodeArgs& a, const G& contr
                 if (!live[b])
                     continue;
                 const int niy = ny0 + r0 + b * T::RS;
-                double un = 0.0, vn = 0.0;
-                double dx = 0.0, dy = 0.0;
-                if (!dir[b]) {
-                    forEachAdjacentXY<CG, true>(nix, niy, a.nx, a.ny, [&](int ex, int ey, int j) {
-                        const int le = (ex - ex0 + 1) + T::HX * (ey - ey0 + 1);
-                        dx -= static_cast<double>(contrib(le, j, 0));
-                        dy -= static_cast<double>(contrib(le, j, 1));
-                    });
-                }
-                if (P::kAllNodes || !dir[b])
-                    pol.update(a, in[b], nix + row * niy, dir[b], dx, dy, un, vn);
-                uOut[nix + row * niy] = un;
-                vOut[nix + row * niy] = vn;
+                double dx, dy, un, vn;
+                nodeDivergence<CG>(
+                    nix, niy, a.nx, a.ny, [&](int ex, int ey) { return (ex - ex0 + 1) + T::HX * (ey - ey0 + 1); },
+                    contrib, dx, dy);
+                pol.update(a, in[b], nix + row * niy, dir[b], P::kAllNodes && dir[b] ? 0.0 : dx,
+                    P::kAllNodes && dir[b] ? 0.0 : dy, un, vn);
+                uOut[nix + row * niy] = dir[b] ? 0.0 : un;
+                vOut[nix + row * niy] = dir[b] ? 0.0 : vn;
             }
         }
     }
@@ -1874,18 +1956,13 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
                 continue;
             const int i = threadIdx.x + b * T::BLOCK;
             const int nix = x0 + i % T::NW, niy = y0 + i / T::NW;
-            double un = 0.0, vn = 0.0;
-            if (!dir[bb]) {
-                double dx = 0.0, dy = 0.0;
-                forEachAdjacentXY<CG, true>(nix, niy, a.nx, a.ny, [&](int exa, int eya, int j) {
-                    const int le = (exa - ex0 + 2) + T::W1 * (eya - ey0 + 2);
-                    dx -= static_cast<double>(contrib[le][j][0]);
-                    dy -= static_cast<double>(contrib[le][j][1]);
-                });
-                momentumFrozen(a, in[bb], dx, dy, un, vn);
-            }
-            uS[i] = un;
-            vS[i] = vn;
+            double dx, dy, un, vn;
+            nodeDivergence<CG>(
+                nix, niy, a.nx, a.ny, [&](int c, int r) { return (c - ex0 + 2) + T::W1 * (r - ey0 + 2); },
+                [&](int le, int j, int c) { return contrib[le][j][c]; }, dx, dy);
+            momentumFrozen(a, in[bb], dx, dy, un, vn);
+            uS[i] = dir[bb] ? 0.0 : un;
+            vS[i] = dir[bb] ? 0.0 : vn;
         }
     }
     __syncthreads();
@@ -2061,36 +2138,6 @@ __device__ __forceinline__ double strainGauss(const ElemArgs& a, const double* g
     }
     return rden;
 }
-// Land elements keep their stored strain: their Gauss-point values replace the velocity's
-// in a branch taken by whole waves (no divergent control flow around the element update).
-template <int CG>
-__device__ __forceinline__ void landStrainGauss(const ElemArgs& a, int e, double* x11, double* x12, double* x22)
-{
-    using L = GeoLayout<CG>;
-    constexpr int S = L::S, NG = L::G;
-    const uint32_t off = static_cast<uint32_t>(e) * 8u;
-    const bool land = !a.ocean[e];
-    if (__builtin_amdgcn_ballot_w64(land) == 0)
-        return;
-    double* const x[3] = { x11, x12, x22 };
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        double s[S];
-#pragma unroll
-        for (int k = 0; k < S; ++k)
-            s[k] = ldAt(a.eps + (c * S + k) * static_cast<size_t>(a.ne), off);
-#pragma unroll
-        for (int q = 0; q < NG * NG; ++q) {
-            double bd[8];
-            dgBasisAt(gauss_point(NG, q % NG) - 0.5, gauss_point(NG, q / NG) - 0.5, bd);
-            double g = 0;
-#pragma unroll
-            for (int k = 0; k < S; ++k)
-                g += s[k] * bd[k];
-            x[c][q] = land ? g : x[c][q];
-        }
-    }
-}
 // The stored strain of the ocean elements from the geometry (the strain output before the
 // last subcycle of a run on a general mesh); land elements keep theirs.
 template <int CG, bool SPH> __global__ __launch_bounds__(kBlock) void k_strain_geom(ElemArgs a, const double* geo)
@@ -2155,7 +2202,7 @@ __device__ __forceinline__ void elementGeomUpdate(const ElemArgs& a, const doubl
             }
         },
         iw);
-    landStrainGauss<CG>(a, e, x11, x12, x22);
+    landStrainGauss<CG, double>(a, e, x11, x12, x22);
     const uint32_t offS = after(after(after(off, x11[Q - 1]), x12[Q - 1]), x22[Q - 1]);
     double k11 = 0, k12 = 0, k22 = 0;
 #pragma unroll
@@ -3206,7 +3253,7 @@ __device__ __forceinline__ void bbmElementGeom(const ElemArgs& a, const BrittleA
             a, geo, e, x11, x12, x22, [&](int q, double w, double, double) { iW[q] = w; },
             [&](int q) { return iW[q]; });
     }
-    landStrainGauss<CG>(a, e, x11, x12, x22);
+    landStrainGauss<CG, double>(a, e, x11, x12, x22);
     // the point arithmetic, h and A per Gauss row
     {
         const uint32_t offH = after(after(after(off, x11[Q - 1]), x12[Q - 1]), x22[Q - 1]);
