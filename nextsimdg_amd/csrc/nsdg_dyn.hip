@@ -951,12 +951,11 @@ template <> __device__ __forceinline__ const float* strengthOf<float>(const Elem
 // Land elements keep their stored strain: its Gauss-point values replace the velocity's in
 // a branch taken by whole waves (no divergent control flow around the element update).
 template <int CG, class C>
-__device__ __forceinline__ void landStrainGauss(const ElemArgs& a, int e, C* x11, C* x12, C* x22)
+__device__ __forceinline__ void landStrainGauss(const ElemArgs& a, int e, bool land, C* x11, C* x12, C* x22)
 {
     using L = MomLayout<CG>;
     constexpr int S = L::S, NG = L::G;
     const uint32_t off = static_cast<uint32_t>(e) * 8u;
-    const bool land = ldAt(a.ocean, static_cast<uint32_t>(e)) == 0;
     if (__builtin_amdgcn_ballot_w64(land) == 0)
         return;
     C* const x[3] = { x11, x12, x22 };
@@ -987,9 +986,12 @@ __device__ __forceinline__ void landStrainGauss(const ElemArgs& a, int e, C* x11
 // old(c, s) the previous stress, component c (11, 12, 22), coefficient s.
 // str(q) gives the ice strength at Gauss point q (row-major, x fastest); by default it is
 // read from the strength table.
-template <int CG, int DG, class R, class C, bool VP, class VEL, class OLD, class STR>
-__device__ __forceinline__ void elementAffineCore(
-    const ElemArgs& a, int e, Acc<C>* acc1, Acc<C>* acc2, Acc<C>* acc3, const VEL& vel, const OLD& old, const STR& str)
+struct Nothing {
+    __device__ __forceinline__ void operator()() const { }
+};
+template <int CG, int DG, class R, class C, bool VP, class VEL, class OLD, class STR, class MID = Nothing>
+__device__ __forceinline__ void elementAffineCore(const ElemArgs& a, int e, bool land, Acc<C>* acc1, Acc<C>* acc2,
+    Acc<C>* acc3, const VEL& vel, const OLD& old, const STR& str, const MID& mid = MID {})
 {
     using L = MomLayout<CG>;
     constexpr int S = L::S, NG = L::G, Q = L::Q, N = L::N, K = CG + 1;
@@ -1052,7 +1054,8 @@ __device__ __forceinline__ void elementAffineCore(
             }
         }
     }
-    landStrainGauss<CG, C>(a, e, x11, x12, x22);
+    landStrainGauss<CG, C>(a, e, land, x11, x12, x22);
+    mid();
     const C DM2 = static_cast<C>(a.DM2);
     // The projected terms sum_q PSI_s(q) w_q / m_s r(q) of each coefficient, summed plainly:
     // in acc (FP64), in t (FP32).
@@ -1132,8 +1135,8 @@ __device__ __forceinline__ void elementAffineCore(
     const R* const Pg = strengthOf<R>(a);
     const size_t ne = a.ne;
     const uint32_t eoff = static_cast<uint32_t>(e) * static_cast<uint32_t>(sizeof(R));
-    elementAffineCore<CG, DG, R, C, VP>(
-        a, e, acc1, acc2, acc3, vel, old, [&](int q) -> C { return ldAt(Pg + q * ne, eoff); });
+    elementAffineCore<CG, DG, R, C, VP>(a, e, ldAt(a.ocean, static_cast<uint32_t>(e)) == 0, acc1, acc2, acc3, vel,
+        old, [&](int q) -> C { return ldAt(Pg + q * ne, eoff); });
 }
 // The element update from the state in HBM (velocity a.u, a.v; stress of precision R);
 // str(q) as in elementAffineCore.
@@ -1146,7 +1149,7 @@ __device__ __forceinline__ void elementAffineCompute(
     const R* const sig = stressOf<R>(a);
     const uint32_t eoff = static_cast<uint32_t>(e) * static_cast<uint32_t>(sizeof(R));
     elementAffineCore<CG, DG, R, C, VP>(
-        a, e, acc1, acc2, acc3,
+        a, e, ldAt(a.ocean, static_cast<uint32_t>(e)) == 0, acc1, acc2, acc3,
         [&](double* lu, double* lv) {
             const int ix = e % a.nx, iy = e / a.nx, row = CG * a.nx + 1;
             const uint32_t noff = static_cast<uint32_t>(CG * row * iy + CG * ix) * 8u;
@@ -1818,9 +1821,20 @@ template <int CG, int DG> __global__ __launch_bounds__(kBlock) void k_residual_f
 // k_mevp_fused, in the same order, from the same operands (a halo value identically in
 // every tile that computes it); the compiler may still fuse a multiply-add differently
 // in the two kernels, which moves a value by an ulp.
-// FP64: 13 x 13 owned elements on 256 threads (51 KB of LDS: three blocks per CU). FP32,
-// bound by instruction issue and with half the LDS per value: 29 x 13 on 512 threads, 2.47
-// element updates per owned element and two subcycles instead of 2.67.
+// FP64: 13 x 13 owned elements on 256 threads. FP32, bound by instruction issue and with
+// half the LDS per value: 29 x 13 on 512 threads, 2.47 element updates per owned element and
+// two subcycles instead of 2.67.
+// FP64 is bound by how much of its memory traffic overlaps its arithmetic: a block alone
+// issues for 8 us and took 18. Every wait for a load covers the loads issued before it
+// (they return in order), so the block issues them in the order of their use, well ahead:
+// the node velocities (coalesced, into an LDS window that the element and node updates
+// share), the strength and the nodes' frozen terms at the start, the previous stress between
+// the strain and the rheology. Strength and frozen terms stay in registers for sub-step 2
+// (252 VGPRs, 68 KB of LDS: two blocks per CU) instead of being read again by three blocks
+// of 160 VGPRs, each phase waiting for its own loads. Per launch: 24 x 24 box 15.8 -> 14.6
+// us, CG1 128 x 128 8.1 -> 7.2, 2048 x 2048 1106 -> 975, 512 x 512 70.6 -> 70.0 (its 1600
+// tiles are 3.1 rounds of 512 blocks). The same registers filled in another order, frozen
+// terms first, took 96 us at 512 x 512.
 template <int CG, class R> struct PairTile {
     static constexpr int TX = sizeof(R) == 8 ? 13 : 29, TY = 13;
     static constexpr int W1 = TX + 3, H1 = TY + 3;          // sub-step 1 elements
@@ -1864,7 +1878,7 @@ struct MevpNodeWindow {
 // use the rounded values; the node update stays FP64).
 template <int CG, int DG, class R>
 __global__ __launch_bounds__((PairTile<CG, R>::BLOCK))
-__attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(FusedArgs f)
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : 1))) void k_mevp_pair(FusedArgs f)
 {
     using T = PairTile<CG, R>;
     constexpr int N = T::N, S = cg2dgstress(CG), K = CG + 1;
@@ -1874,6 +1888,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
     __shared__ R contribRaw[CWORDS > SWORDS ? CWORDS : SWORDS];
     auto& contrib = *reinterpret_cast<R(*)[T::W1 * T::H1][N][2]>(contribRaw);
     __shared__ double uS[NWH], vS[NWH];
+    constexpr bool kKeep = sizeof(R) == 8;
+    // FP64: the nodes of the sub-step 1 elements, u^k and v^k
+    constexpr int NW0 = CG * T::W1 + 1, NWH0 = NW0 * (CG * T::H1 + 1), NB0 = (NWH0 + T::BLOCK - 1) / T::BLOCK;
+    __shared__ double u0S[kKeep ? NWH0 : 1], v0S[kKeep ? NWH0 : 1];
     const NodeArgs& a = f.n;
     const int tilesX = (a.nx + T::TX - 1) / T::TX, tilesY = (a.ny + T::TY - 1) / T::TY;
     const int tile = xcdTile(blockIdx.x, tilesX * tilesY);
@@ -1886,13 +1904,27 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
     const int ex = ex0 - 2 + lx, ey = ey0 - 2 + ly;
     const bool inDomain = ex >= 0 && ex < a.nx && ey >= 0 && ey < a.ny;
     const int e = inDomain ? ex + a.nx * ey : 0;
+    const bool land = ldAt(a.ocean, static_cast<uint32_t>(e)) == 0;
     R s11[S], s12[S], s22[S]; // sigma^(k+1) of this thread's element
-    // the element's Gauss-point strength for sub-step 1. Sub-step 2 reads it again in FP64
-    // (from the L2): the 18 VGPRs it frees give the FP64 pass a third block per CU
-    // (occupancy 3, 168 VGPRs; LDS 3 x 50 KB). FP32 keeps it in registers.
+    // the element's Gauss-point strength, for both sub-steps
     constexpr int Q = MomLayout<CG>::Q;
     R pk[Q];
-    if (inDomain) {
+    // FP64: node velocities, strength, then the frozen terms of this thread's nodes
+    double2 fzOcn[kKeep ? NB : 1], fzCf[kKeep ? NB : 1], fzQf[kKeep ? NB : 1];
+    bool fzLive[NB], fzDir[NB];
+    double u0[kKeep ? NB0 : 1], v0[kKeep ? NB0 : 1];
+    if constexpr (kKeep) {
+#pragma unroll
+        for (int b = 0; b < NB0; ++b) {
+            const int i = threadIdx.x + b * T::BLOCK;
+            const int nix = x0 - CG + i % NW0, niy = y0 - CG + i / NW0;
+            const bool in = nix >= 0 && nix <= CG * a.nx && niy >= 0 && niy <= CG * a.ny;
+            const uint32_t n = in ? static_cast<uint32_t>(nix + row * niy) * 8u : 0u;
+            u0[b] = ldAt(a.u, n);
+            v0[b] = ldAt(a.v, n);
+        }
+    }
+    {
         const R* const Pg = strengthOf<R>(f.e);
         const uint32_t eoff = static_cast<uint32_t>(e) * static_cast<uint32_t>(sizeof(R));
 #pragma unroll
@@ -1900,13 +1932,28 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
             pk[q] = ldAt(Pg + static_cast<uint32_t>(q) * static_cast<uint32_t>(f.e.ne), eoff); // < 2^32: ne < 2^29
     }
     const auto kept = [&](int q) -> R { return pk[q]; };
-    const auto strength2 = [&](int q) -> R {
-        if constexpr (sizeof(R) == 8)
-            return ldAt(strengthOf<R>(f.e) + static_cast<uint32_t>(q) * static_cast<uint32_t>(f.e.ne),
-                static_cast<uint32_t>(e) * static_cast<uint32_t>(sizeof(R)));
-        else
-            return pk[q];
-    };
+    if constexpr (kKeep) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int i = threadIdx.x + b * T::BLOCK;
+            const int nix = x0 + i % T::NW, niy = y0 + i / T::NW;
+            fzLive[b] = i < NWH && nix >= 0 && nix <= CG * a.nx && niy >= 0 && niy <= CG * a.ny;
+            const uint32_t n = fzLive[b] ? static_cast<uint32_t>(nix + row * niy) : 0u;
+            fzDir[b] = ldAt(a.dirNode, n) != 0;
+            fzOcn[b] = ld2At(a.ocn, n * 16u);
+            fzCf[b] = ld2At(a.cf, n * 16u);
+            fzQf[b] = ld2At(a.qf, n * 16u);
+        }
+#pragma unroll
+        for (int b = 0; b < NB0; ++b) {
+            const int i = threadIdx.x + b * T::BLOCK;
+            if (i < NWH0) {
+                u0S[i] = u0[b];
+                v0S[i] = v0[b];
+            }
+        }
+        __syncthreads();
+    }
     {
         R tx[N], ty[N];
 #pragma unroll
@@ -1914,14 +1961,34 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
             tx[j] = ty[j] = 0;
         if (inDomain) {
             Acc<R> acc1[S], acc2[S], acc3[S];
-            elementAffineCompute<CG, DG, R, R, false>(f.e, e, acc1, acc2, acc3, kept);
+            R sOld[kKeep ? 3 * S : 1];
+            if constexpr (kKeep)
+                elementAffineCore<CG, DG, R, R, false>(
+                    f.e, e, land, acc1, acc2, acc3,
+                    [&](double* lu, double* lv) {
+#pragma unroll
+                        for (int r = 0; r < K; ++r)
+#pragma unroll
+                            for (int c = 0; c < K; ++c) {
+                                lu[c + K * r] = u0S[CG * lx + c + NW0 * (CG * ly + r)];
+                                lv[c + K * r] = v0S[CG * lx + c + NW0 * (CG * ly + r)];
+                            }
+                    },
+                    [&](int c, int k) -> R { return sOld[c * S + k]; }, kept,
+                    [&] {
+#pragma unroll
+                        for (int k = 0; k < 3 * S; ++k)
+                            sOld[k] = ldAt(stressOf<R>(f.e) + k * static_cast<size_t>(a.ne), static_cast<uint32_t>(e) * 8u);
+                    });
+            else
+                elementAffineCompute<CG, DG, R, R, false>(f.e, e, acc1, acc2, acc3, kept);
 #pragma unroll
             for (int k = 0; k < S; ++k) {
                 s11[k] = storeValue<R>(acc1[k], e, 0 * S + k, f.e.iter);
                 s12[k] = storeValue<R>(acc2[k], e, 1 * S + k, f.e.iter);
                 s22[k] = storeValue<R>(acc3[k], e, 2 * S + k, f.e.iter);
             }
-            if (a.ocean[e])
+            if (!land)
                 divergenceAffineFrom<CG, R>(a, s11, s12, s22, tx, ty);
         }
 #pragma unroll
@@ -1931,38 +1998,56 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
         }
     }
     __syncthreads();
-    // sub-step 1, the nodes of the inner elements (within the domain) into LDS, in batches
-    // of NBB nodes per thread (each batch's frozen terms loaded before its gathers, for
-    // Dirichlet nodes too, so that the loads do not wait for the Dirichlet flag)
-    constexpr int NBB = 2;
+    // sub-step 1, the nodes of the inner elements (within the domain) into LDS
+    if constexpr (kKeep) {
 #pragma unroll
-    for (int b0 = 0; b0 < NB; b0 += NBB) {
-        NodeFz in[NBB];
-        bool live[NBB], dir[NBB];
-#pragma unroll
-        for (int bb = 0; bb < NBB; ++bb) {
-            const int i = threadIdx.x + (b0 + bb) * T::BLOCK;
-            const int nix = x0 + i % T::NW, niy = y0 + i / T::NW;
-            live[bb] = b0 + bb < NB && i < NWH && nix >= 0 && nix <= CG * a.nx && niy >= 0 && niy <= CG * a.ny;
-            const int n = nix + row * niy;
-            dir[bb] = live[bb] ? a.dirNode[n] != 0 : true;
-            if (live[bb])
-                loadFrozenAt(a, static_cast<uint32_t>(n), in[bb]);
-        }
-#pragma unroll
-        for (int bb = 0; bb < NBB; ++bb) {
-            const int b = b0 + bb;
-            if (!live[bb])
-                continue;
+        for (int b = 0; b < NB; ++b) {
             const int i = threadIdx.x + b * T::BLOCK;
             const int nix = x0 + i % T::NW, niy = y0 + i / T::NW;
+            if (!fzLive[b])
+                continue;
             double dx, dy, un, vn;
             nodeDivergence<CG>(
                 nix, niy, a.nx, a.ny, [&](int c, int r) { return (c - ex0 + 2) + T::W1 * (r - ey0 + 2); },
                 [&](int le, int j, int c) { return contrib[le][j][c]; }, dx, dy);
-            momentumFrozen(a, in[bb], dx, dy, un, vn);
-            uS[i] = dir[bb] ? 0.0 : un;
-            vS[i] = dir[bb] ? 0.0 : vn;
+            const int l = CG + i % T::NW + NW0 * (CG + i / T::NW);
+            momentumFrozen(a, NodeFz { u0S[l], v0S[l], fzOcn[b], fzCf[b], fzQf[b] }, dx, dy, un, vn);
+            uS[i] = fzDir[b] ? 0.0 : un;
+            vS[i] = fzDir[b] ? 0.0 : vn;
+        }
+    } else {
+        // FP32: in batches of NBB nodes per thread (each batch's frozen terms loaded before its
+        // gathers, for Dirichlet nodes too, so that the loads do not wait for the Dirichlet flag)
+        constexpr int NBB = 2;
+#pragma unroll
+        for (int b0 = 0; b0 < NB; b0 += NBB) {
+            NodeFz in[NBB];
+            bool live[NBB], dir[NBB];
+#pragma unroll
+            for (int bb = 0; bb < NBB; ++bb) {
+                const int i = threadIdx.x + (b0 + bb) * T::BLOCK;
+                const int nix = x0 + i % T::NW, niy = y0 + i / T::NW;
+                live[bb] = b0 + bb < NB && i < NWH && nix >= 0 && nix <= CG * a.nx && niy >= 0 && niy <= CG * a.ny;
+                const int n = nix + row * niy;
+                dir[bb] = live[bb] ? a.dirNode[n] != 0 : true;
+                if (live[bb])
+                    loadFrozenAt(a, static_cast<uint32_t>(n), in[bb]);
+            }
+#pragma unroll
+            for (int bb = 0; bb < NBB; ++bb) {
+                const int b = b0 + bb;
+                if (!live[bb])
+                    continue;
+                const int i = threadIdx.x + b * T::BLOCK;
+                const int nix = x0 + i % T::NW, niy = y0 + i / T::NW;
+                double dx, dy, un, vn;
+                nodeDivergence<CG>(
+                    nix, niy, a.nx, a.ny, [&](int c, int r) { return (c - ex0 + 2) + T::W1 * (r - ey0 + 2); },
+                    [&](int le, int j, int c) { return contrib[le][j][c]; }, dx, dy);
+                momentumFrozen(a, in[bb], dx, dy, un, vn);
+                uS[i] = dir[bb] ? 0.0 : un;
+                vS[i] = dir[bb] ? 0.0 : vn;
+            }
         }
     }
     __syncthreads();
@@ -1989,7 +2074,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
             const int bx = CG * (ex - ex0 + 1), by = CG * (ey - ey0 + 1); // first node in the window
             Acc<R> acc1[S], acc2[S], acc3[S];
             elementAffineCore<CG, DG, R, R, false>(
-                f.e, e, acc1, acc2, acc3,
+                f.e, e, land, acc1, acc2, acc3,
                 [&](double* lu, double* lv) {
 #pragma unroll
                     for (int r = 0; r < K; ++r)
@@ -1999,7 +2084,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
                             lv[c + K * r] = vS[bx + c + T::NW * (by + r)];
                         }
                 },
-                [&](int c, int k) -> R { return sigS[(c * S + k) * NI + le2]; }, strength2);
+                [&](int c, int k) -> R { return sigS[(c * S + k) * NI + le2]; }, kept);
             R n11[S], n12[S], n22[S];
 #pragma unroll
             for (int k = 0; k < S; ++k) {
@@ -2014,7 +2099,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
                 else
                     storeTensorAt<S>(f.sigFOut, a.ne, eoff, n11, n12, n22);
             }
-            if (a.ocean[e])
+            if (!land)
                 divergenceAffineFrom<CG, R>(a, n11, n12, n22, tx, ty);
         }
         __syncthreads(); // every parked stress is read before the contributions overwrite it
@@ -2027,9 +2112,29 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1))) void k_mevp_pair(Fu
         }
     }
     __syncthreads();
-    nodeTileUpdate<CG, typename T::Inner, MevpNodeWindow>(
-        a, [&](int le, int j, int c) { return contrib[le][j][c]; }, ex0, ey0, f.uOut, f.vOut,
-        MevpNodeWindow { uS, vS, x0, y0, T::NW });
+    if constexpr (kKeep) {
+        const int W = (ex0 + T::TX >= a.nx) ? CG * a.nx + 1 - CG * ex0 : CG * T::TX;
+        const int H = (ey0 + T::TY >= a.ny) ? CG * a.ny + 1 - CG * ey0 : CG * T::TY;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int i = threadIdx.x + b * T::BLOCK;
+            const int c = i % T::NW - CG, r = i / T::NW - CG;
+            if (i >= NWH || c < 0 || r < 0 || c >= W || r >= H)
+                continue;
+            const int nix = CG * ex0 + c, niy = CG * ey0 + r, n = nix + row * niy;
+            double dx, dy, un, vn;
+            nodeDivergence<CG>(
+                nix, niy, a.nx, a.ny, [&](int c, int r) { return (c - ex0 + 1) + T::W2 * (r - ey0 + 1); },
+                [&](int le, int j, int c) { return contrib[le][j][c]; }, dx, dy);
+            momentumFrozen(a, NodeFz { uS[i], vS[i], fzOcn[b], fzCf[b], fzQf[b] }, dx, dy, un, vn);
+            f.uOut[n] = fzDir[b] ? 0.0 : un;
+            f.vOut[n] = fzDir[b] ? 0.0 : vn;
+        }
+    } else {
+        nodeTileUpdate<CG, typename T::Inner, MevpNodeWindow>(
+            a, [&](int le, int j, int c) { return contrib[le][j][c]; }, ex0, ey0, f.uOut, f.vOut,
+            MevpNodeWindow { uS, vS, x0, y0, T::NW });
+    }
 }
 
 // PSI_s(q) w_q / m_s, the projection of Gauss-point values on the reference element.
@@ -2202,7 +2307,7 @@ __device__ __forceinline__ void elementGeomUpdate(const ElemArgs& a, const doubl
             }
         },
         iw);
-    landStrainGauss<CG, double>(a, e, x11, x12, x22);
+    landStrainGauss<CG, double>(a, e, !a.ocean[e], x11, x12, x22);
     const uint32_t offS = after(after(after(off, x11[Q - 1]), x12[Q - 1]), x22[Q - 1]);
     double k11 = 0, k12 = 0, k22 = 0;
 #pragma unroll
@@ -3253,7 +3358,7 @@ __device__ __forceinline__ void bbmElementGeom(const ElemArgs& a, const BrittleA
             a, geo, e, x11, x12, x22, [&](int q, double w, double, double) { iW[q] = w; },
             [&](int q) { return iW[q]; });
     }
-    landStrainGauss<CG, double>(a, e, x11, x12, x22);
+    landStrainGauss<CG, double>(a, e, !a.ocean[e], x11, x12, x22);
     // the point arithmetic, h and A per Gauss row
     {
         const uint32_t offH = after(after(after(off, x11[Q - 1]), x12[Q - 1]), x22[Q - 1]);
