@@ -154,6 +154,12 @@ __device__ __forceinline__ double quotient(double a, double b)
     const double r = reciprocal(b), q = a * r;
     return fma(fma(-b, q, a), r, q);
 }
+// x, not to be computed behind a branch on the condition that selects it.
+__device__ __forceinline__ double computed(double x)
+{
+    asm("" : "+v"(x));
+    return x;
+}
 // One third-order step: the estimate's error cubed is below the rounding.
 __device__ __forceinline__ double rsq(double x)
 {
@@ -2248,9 +2254,11 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : 1))) void k_mevp_pair(Fu
 // g(q) / W_q, with g the J-weighted velocity gradients, sum-factorised from the 1-D CG
 // basis. keep(q, iW, cl, sl) receives 1 / W_q and the latitude's cosine and sine; iw(q)
 // gives 1 / W_q back. Returns 1 / sum n^2 / W.
-template <int CG, bool SPH, class KEEP, class IW>
+// then() runs after the strain's own loads are issued: what the caller loads there
+// returns while the strain is formed.
+template <int CG, bool SPH, class KEEP, class IW, class THEN = Nothing>
 __device__ __forceinline__ double strainGauss(const ElemArgs& a, const double* geo, int e, double* x11, double* x12,
-    double* x22, const KEEP& keep, const IW& iw)
+    double* x22, const KEEP& keep, const IW& iw, const THEN& then = THEN {})
 {
     using L = GeoLayout<CG>;
     constexpr int NG = L::G, N = cgdofs(CG), K = CG + 1;
@@ -2270,6 +2278,12 @@ __device__ __forceinline__ double strainGauss(const ElemArgs& a, const double* g
                 lv[c + K * r] = ldAt(a.v + c + r * row, noff);
             }
     }
+    double lat[SPH ? 2 * L::Q : 1]; // cos and sin of the latitude
+    if constexpr (SPH)
+#pragma unroll
+        for (int k = 0; k < 2 * L::Q; ++k)
+            lat[k] = ldAt(g1 + (L::CL + k) * ne, off);
+    then();
     double den = 0, k11 = 0, k12 = 0, k22 = 0;
     double Iu[K][NG], Du[K][NG], Iv[K][NG], Dv[K][NG];
     cgColumns<CG>(lu, Iu, Du);
@@ -2283,8 +2297,7 @@ __device__ __forceinline__ double strainGauss(const ElemArgs& a, const double* g
         for (int gx = 0; gx < NG; ++gx) {
             const int q = gx + NG * gy;
             const double uxi = ruxi[gx], ueta = rueta[gx], vxi = rvxi[gx], veta = rveta[gx];
-            const double cl = SPH ? ldAt(g1 + (L::CL + q) * ne, off) : 1.0;
-            const double sl = SPH ? ldAt(g1 + (L::SL + q) * ne, off) : 0.0;
+            const double cl = SPH ? lat[SPH ? q : 0] : 1.0, sl = SPH ? lat[SPH ? L::Q + q : 0] : 0.0;
             const GaussGeom gg = gaussGeom<NG, SPH>(map, gx, gy, cl, sl);
             double g11 = gg.a * uxi - gg.b * ueta;
             const double g22 = gg.c * veta - gg.d * vxi;
@@ -2356,6 +2369,7 @@ template <int CG, bool SPH> __global__ __launch_bounds__(kBlock) void k_strain_g
 template <int CG, bool SPH> struct GeoColumn {
     static constexpr int Q = GeoLayout<CG>::Q, CL = Q - 1, SL = 2 * Q - 1, K = SPH ? 3 * Q - 1 : Q - 1;
 };
+// The strength and the previous stress are loaded ahead of the strain.
 template <int CG, bool SPH, class COL>
 __device__ __forceinline__ void elementGeomUpdate(const ElemArgs& a, const double* geo, int e, double* s11,
     double* s12, double* s22, const COL& col)
@@ -2363,6 +2377,8 @@ __device__ __forceinline__ void elementGeomUpdate(const ElemArgs& a, const doubl
     using L = GeoLayout<CG>;
     using C = GeoColumn<CG, SPH>;
     constexpr int S = L::S, NG = L::G, Q = L::Q;
+    const bool land = ldAt(a.ocean, static_cast<uint32_t>(e)) == 0;
+    double Pg[Q], old[3 * S];
     const size_t ne = a.ne;
     const uint32_t off = static_cast<uint32_t>(e) * 8u;
     double x11[Q], x12[Q], x22[Q], iWlast = 0.0;
@@ -2379,9 +2395,16 @@ __device__ __forceinline__ void elementGeomUpdate(const ElemArgs& a, const doubl
                 col(C::SL + q) = sl;
             }
         },
-        iw);
-    landStrainGauss<CG, double>(a, e, !a.ocean[e], x11, x12, x22);
-    const uint32_t offS = after(after(after(off, x11[Q - 1]), x12[Q - 1]), x22[Q - 1]);
+        iw,
+        [&] {
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+                Pg[q] = ldAt(a.Pg + q * ne, off);
+#pragma unroll
+            for (int k = 0; k < 3 * S; ++k)
+                old[k] = ldAt(a.sig + k * ne, off);
+        });
+    landStrainGauss<CG, double>(a, e, land, x11, x12, x22);
     double k11 = 0, k12 = 0, k22 = 0;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
@@ -2390,7 +2413,7 @@ __device__ __forceinline__ void elementGeomUpdate(const ElemArgs& a, const doubl
         double w = 0.5 * a.invAlpha;
         if constexpr (SPH)
             w *= reciprocal(col(C::CL + q));
-        const double h = ldAt(a.Pg + q * ne, offS) * w; // P / (2 alpha), as in elementAffineCore
+        const double h = Pg[q] * w; // P / (2 alpha), as in elementAffineCore
         const double c = h * rsq(X), c2 = 0.5 * c;
         const double t = c * p - h, d = c2 * m;
         const double n = complementAt<CG>(q % NG, q / NG);
@@ -2415,14 +2438,12 @@ __device__ __forceinline__ void elementGeomUpdate(const ElemArgs& a, const doubl
     projectionMoments<CG>(x11, s11);
     projectionMoments<CG>(x12, s12);
     projectionMoments<CG>(x22, s22);
-    // the previous stress is read only now
-    const uint32_t offM = after(after(after(off, s11[S - 1]), s12[S - 1]), s22[S - 1]);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const double k = momentScale(CG, s);
-        s11[s] = ldAt(a.sig + (0 * S + s) * ne, offM) * a.relax + k * s11[s];
-        s12[s] = ldAt(a.sig + (1 * S + s) * ne, offM) * a.relax + k * s12[s];
-        s22[s] = ldAt(a.sig + (2 * S + s) * ne, offM) * a.relax + k * s22[s];
+        s11[s] = old[0 * S + s] * a.relax + k * s11[s];
+        s12[s] = old[1 * S + s] * a.relax + k * s12[s];
+        s22[s] = old[2 * S + s] * a.relax + k * s22[s];
     }
 }
 // Weak-divergence contributions of one element (CGDynamicsKernel.cpp:339-398 with the
@@ -2497,12 +2518,16 @@ __device__ __forceinline__ void divergenceGeomFrom(const double* geo, size_t ne,
 // One whole mEVP subcycle in one pass over a general (non-affine or spherical) mesh without
 // periodic segments, FP64: k_mevp_fused's tiles, halo and node phase, with the element
 // update and the divergence computed from the streamed geometry instead of literals.
-// Bound by its traffic and the latency of its dependent loads: without the inverse mass
-// (the projection goes through the Gauss weights) and with the latitudes kept in LDS from
-// the strain to the divergence it runs without a spill at three blocks per CU (168 VGPRs
-// on the sphere, 53 KB of LDS). 512 x 512 spherical patch: 86.6 -> 64.4 us per subcycle.
+// Bound by its traffic, near the copy rate on large meshes, and by the latency of one block
+// on small ones: nothing of an inverse mass is streamed (the projection goes through the
+// Gauss weights), the latitudes stay in LDS from the strain to the divergence, and all that
+// the element reads is issued before the strain (182 VGPRs, two blocks per CU; three blocks
+// of 168 that load strength and stress where they are used: 59.0 and 12.9 us in place of
+// the last figures). Per subcycle, in these steps: 512 x 512 spherical patch 86.6 -> 64.4 ->
+// 61.9 (sum factorisations) -> 58.2 us, 154 x 121 16.5 -> 13.4 -> 12.5 us. Loading the
+// first nodes' terms before the divergence as well was slower (60.0 us).
 template <int CG, int DG, bool SPH>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CG == 2 ? 3 : 4))) void k_mevp_fused_geom(FusedArgs f)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_mevp_fused_geom(FusedArgs f)
 {
     using T = FusedTile<CG>;
     constexpr int N = T::N, S = cg2dgstress(CG);
@@ -2938,7 +2963,8 @@ __device__ __forceinline__ void bbmPoint(const BrittleArgs& b, double hg, double
     const double sc = -sn0;
     const bool part = sc > 1e-200;
     const double tn = part ? tv * sc : tv;
-    const double mult = sn0 < 0.0 && Pmax >= sc ? 1.0 : quotient(tn, tn + dt * (part ? sc - Pmax : 1.0));
+    const double ratio = computed(quotient(tn, tn + dt * (part ? sc - Pmax : 1.0)));
+    const double mult = sn0 < 0.0 && Pmax >= sc ? 1.0 : ratio;
     const double E = hg * b.young * dg * expC;
     const double Du = b.duFac * E;
     y11 = (y11 + Du * (x11 + nu * x22)) * mult;
@@ -2952,7 +2978,8 @@ __device__ __forceinline__ void bbmPoint(const BrittleArgs& b, double hg, double
     // first, so one division serves both branches
     const bool compressive = sn < -cstr, shear = tau + b.tanPhi * sn > 0.0;
     const double num = compressive ? -cstr : cohesion, den = compressive ? sn : tau + b.tanPhi * sn;
-    const double dcrit = fmin(compressive || shear ? quotient(num, den) : 1.0, 1.0);
+    const double crit = computed(quotient(num, den));
+    const double dcrit = fmin(compressive || shear ? crit : 1.0, 1.0);
     const double relax = (1.0 - dcrit) * (b.dtOverT * squareRoot(E));
     dg -= dg * relax;
     y11 -= y11 * relax;
@@ -3092,28 +3119,42 @@ template <int DG, int NG, class AT> __device__ __forceinline__ void dgAtGauss(co
             at(gx + NG * gy, v[gx]);
     }
 }
-template <int DG, int NG, class GP>
-__device__ __forceinline__ void bbmInterpolateToGauss(const double* f, size_t ne, int e, int r, GP& gp)
-{
-    double c[DG];
+// What the brittle update of an element reads besides its velocities: loaded at once, ahead
+// of the strain, so that one wait covers it (the loads return while the strain is formed).
+template <int CG, int DG> struct BrittleState {
+    static constexpr int S = MomLayout<CG>::S, NG = MomLayout<CG>::G;
+    double s[3][S], d[DG], h[DG], A[DG];
+    __device__ __forceinline__ void load(const ElemArgs& a, const BrittleArgs& b, int e)
+    {
+        const size_t ne = a.ne;
+        const uint32_t off = static_cast<uint32_t>(e) * 8u;
 #pragma unroll
-    for (int i = 0; i < DG; ++i)
-        c[i] = ldAt(f + i * ne, static_cast<uint32_t>(e) * 8u);
-    dgAtGauss<DG, NG>(c, [&](int q, double v) { gp(4 * q + r) = v; });
-}
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+                s[c][k] = ldAt(a.sig + (c * S + k) * ne, off);
+#pragma unroll
+        for (int i = 0; i < DG; ++i) {
+            d[i] = ldAt(b.damageIn + i * ne, off);
+            h[i] = ldAt(a.h + i * ne, off);
+            A[i] = ldAt(a.A + i * ne, off);
+        }
+    }
+    // the stress and damage at the Gauss points into the thread's column
+    template <class GP> __device__ __forceinline__ void stage(const GP& gp) const
+    {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            dgAtGauss<S, NG>(s[c], [&](int q, double v) { gp(4 * q + c) = v; });
+        dgAtGauss<DG, NG>(d, [&](int q, double v) { gp(4 * q + 3) = v; });
+    }
+};
 // The point arithmetic at every Gauss point, h and A evaluated per Gauss row.
 template <int CG, int DG, bool POW5, class GP>
-__device__ __forceinline__ void bbmGaussLoop(const ElemArgs& a, const BrittleArgs& b, uint32_t off, const double* x11,
-    const double* x12, const double* x22, const GP& gp)
+__device__ __forceinline__ void bbmGaussLoop(const BrittleArgs& b, const double* hc, const double* ac,
+    const double* x11, const double* x12, const double* x22, const GP& gp)
 {
     constexpr int NG = MomLayout<CG>::G;
-    const size_t ne = a.ne;
-    double hc[DG], ac[DG];
-#pragma unroll
-    for (int i = 0; i < DG; ++i) {
-        hc[i] = ldAt(a.h + i * ne, off);
-        ac[i] = ldAt(a.A + i * ne, off);
-    }
 #pragma unroll
     for (int gy = 0; gy < NG; ++gy) {
         const double Y = gauss_point(NG, gy) - 0.5;
@@ -3146,14 +3187,10 @@ __device__ __forceinline__ void bbmElementAffine(const ElemArgs& a, const Brittl
     double* acc2, double* acc3, double* accD, GP&& gp)
 {
     using L = MomLayout<CG>;
-    constexpr int S = L::S, NG = L::G, Q = L::Q, N = L::N, K = CG + 1;
-    const size_t ne = a.ne;
+    constexpr int S = L::S, Q = L::Q, N = L::N, K = CG + 1;
     const bool land = ldAt(a.ocean, static_cast<uint32_t>(e)) == 0;
-    bbmInterpolateToGauss<S, NG>(a.sig + 0 * S * ne, ne, e, 0, gp);
-    bbmInterpolateToGauss<S, NG>(a.sig + 1 * S * ne, ne, e, 1, gp);
-    bbmInterpolateToGauss<S, NG>(a.sig + 2 * S * ne, ne, e, 2, gp);
-    bbmInterpolateToGauss<DG, NG>(b.damageIn, ne, e, 3, gp);
     double x11[Q], x12[Q], x22[Q];
+    BrittleState<CG, DG> st;
     {
         double lu[N], lv[N];
         const int ix = e % a.nx, iy = e / a.nx, row = CG * a.nx + 1;
@@ -3165,10 +3202,12 @@ __device__ __forceinline__ void bbmElementAffine(const ElemArgs& a, const Brittl
                 lu[c + K * r] = ldAt(a.u + c + r * row, noff);
                 lv[c + K * r] = ldAt(a.v + c + r * row, noff);
             }
+        st.load(a, b, e);
         strainAffine<CG, double>(a, lu, lv, x11, x12, x22);
     }
     landStrainGauss<CG, double>(a, e, land, x11, x12, x22);
-    bbmGaussLoop<CG, DG, POW5>(a, b, static_cast<uint32_t>(e) * 8u, x11, x12, x22, gp);
+    st.stage(gp);
+    bbmGaussLoop<CG, DG, POW5>(b, st.h, st.A, x11, x12, x22, gp);
     const auto project = [&](int c, double* acc, int n) {
         double r[Q], m[8];
 #pragma unroll
@@ -3301,6 +3340,11 @@ struct BrittleFusedArgs {
     double* vOut;
     const double* geo; // GeoLayout tables of a general mesh (k_bbm_fused_geom)
 };
+// Bound by instruction issue and by the latency of its loads at two blocks per CU. 512 x 512:
+// 78.7 -> 71.7 us per substep (sum factorisations, one point loop for ocean and land, short
+// roots) -> 66.5 (all loads ahead of the strain; the two quotients of a point computed
+// before the conditions that select them, so that the points' chains overlap). Loading the
+// first nodes' terms before the divergence was slower (70.0 us).
 template <int CG, int DG, bool POW5>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_bbm_fused(BrittleFusedArgs f)
 {
@@ -3374,20 +3418,18 @@ __device__ __forceinline__ void bbmElementGeom(const ElemArgs& a, const BrittleA
         b.compr = b.comprStrength * scale;
         b.dtOverT = b.dt / (hE * b.tdFac);
     }
-    bbmInterpolateToGauss<S, NG>(a.sig + 0 * S * ne, ne, e, 0, col);
-    bbmInterpolateToGauss<S, NG>(a.sig + 1 * S * ne, ne, e, 1, col);
-    bbmInterpolateToGauss<S, NG>(a.sig + 2 * S * ne, ne, e, 2, col);
-    bbmInterpolateToGauss<DG, NG>(b.damageIn, ne, e, 3, col);
+    const bool land = ldAt(a.ocean, static_cast<uint32_t>(e)) == 0;
     double x11[Q], x12[Q], x22[Q];
+    BrittleState<CG, DG> st;
     {
         double iW[Q];
         strainGauss<CG, SPH>(
             a, geo, e, x11, x12, x22, [&](int q, double w, double, double) { iW[q] = w; },
-            [&](int q) { return iW[q]; });
+            [&](int q) { return iW[q]; }, [&] { st.load(a, bIn, e); });
     }
-    landStrainGauss<CG, double>(a, e, !a.ocean[e], x11, x12, x22);
-    bbmGaussLoop<CG, DG, POW5>(
-        a, b, after(after(after(off, x11[Q - 1]), x12[Q - 1]), x22[Q - 1]), x11, x12, x22, col);
+    landStrainGauss<CG, double>(a, e, land, x11, x12, x22);
+    st.stage(col);
+    bbmGaussLoop<CG, DG, POW5>(b, st.h, st.A, x11, x12, x22, col);
     // projections: the stress through the Gauss weights (strainGauss, and on the sphere of
     // y / cos(lat)), the damage by the packed inverse DG mass
     const double* const g2 = phaseLocal(geo);
@@ -3456,9 +3498,11 @@ __device__ __forceinline__ void bbmElementGeom(const ElemArgs& a, const BrittleA
 }
 // One whole brittle substep in one pass over a general mesh without periodic segments:
 // k_bbm_fused's tiles, halo, staging and node phase with the element update and the
-// divergence computed from the streamed geometry (397 x 263 non-affine box: 41.0 -> 34.8 us
-// per substep without the streamed inverse mass of the stress space).
-template <int CG, int DG, bool POW5, bool SPH> __global__ __launch_bounds__(kBlock) void k_bbm_fused_geom(BrittleFusedArgs f)
+// divergence computed from the streamed geometry. 397 x 263 non-affine box: 41.0 -> 34.8 us
+// per substep without the streamed inverse mass of the stress space, 31.8 with the sum
+// factorisations, short roots and the state loaded ahead of the strain.
+template <int CG, int DG, bool POW5, bool SPH>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_bbm_fused_geom(BrittleFusedArgs f)
 {
     using T = FusedTile<CG>;
     constexpr int N = T::N, S = cg2dgstress(CG), Q = MomLayout<CG>::Q;
