@@ -306,6 +306,45 @@ template <int DG, int SIDE> __device__ __forceinline__ void trace(const double* 
     }
 }
 
+// ---------------------------------------------------------------- DG basis on the Gauss points
+// 1 / m_s, the inverse mass of basis function s on the reference element.
+__device__ __forceinline__ constexpr double invMassRef(int s)
+{
+    return s == 0 ? 1.0 : (s <= 2 ? 12.0 : (s <= 4 ? 180.0 : (s == 5 ? 144.0 : 2160.0)));
+}
+// a0 + a1 X + a2 (X^2 - 1/12) at the Gauss points.
+template <int NG> __device__ __forceinline__ void legendreValues(double a0, double a1, double a2, double* v)
+{
+    const double g = gauss_point(NG, NG - 1) - 0.5;
+    if constexpr (NG == 1) {
+        v[0] = a0;
+    } else if constexpr (NG == 3) {
+        const double e = a0 + (1.0 / 15.0) * a2;
+        v[0] = e - g * a1;
+        v[1] = a0 - (1.0 / 12.0) * a2;
+        v[2] = e + g * a1;
+    } else {
+        v[0] = a0 - g * a1; // two points: the quadratic vanishes there
+        v[1] = a0 + g * a1;
+    }
+}
+// at(q, value) for a DG field with coefficients c (degrees as in dgBasisAt).
+template <int DG, int NG, class AT> __device__ __forceinline__ void dgAtGauss(const double* c, const AT& at)
+{
+    const auto k = [&](int i) { return i < DG ? c[i < DG ? i : 0] : 0.0; };
+    double r0[NG], r1[NG], r2[NG], v[NG];
+    legendreValues<NG>(k(0), k(2), k(4), r0);
+    legendreValues<NG>(k(1), k(5), k(7), r1);
+    legendreValues<NG>(k(3), k(6), 0.0, r2);
+#pragma unroll
+    for (int gy = 0; gy < NG; ++gy) {
+        legendreValues<NG>(r0[gy], r1[gy], r2[gy], v);
+#pragma unroll
+        for (int gx = 0; gx < NG; ++gx)
+            at(gx + NG * gy, v[gx]);
+    }
+}
+
 // ---------------------------------------------------------------- node adjacency
 // Elements sharing CG node (nix, niy) of a degree-CG mesh, visited in the order a
 // two-colour row-stripe scatter adds them: element rows of one parity first, then the

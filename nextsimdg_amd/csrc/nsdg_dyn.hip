@@ -869,10 +869,6 @@ __device__ __forceinline__ void stressLocal(const ElemArgs& a, int e, const doub
 //    m = (1, 1/12, 1/12, 1/180, 1/180, 1/144, 1/2160, 1/2160) on every affine element.
 // Land elements take their strain from the stored coefficients (the reference never
 // updates it).
-__device__ __forceinline__ constexpr double invMassRef(int s)
-{
-    return s == 0 ? 1.0 : (s <= 2 ? 12.0 : (s <= 4 ? 180.0 : (s == 5 ? 144.0 : 2160.0)));
-}
 // The relaxed stress: plain in FP64; in FP32 a (sum, compensation) pair whose exact value
 // is s - c (initSum: Fast2Sum of a + b, exact when |a| >= |b| or a = 0).
 template <class R> struct Acc {
@@ -3089,36 +3085,6 @@ __device__ __forceinline__ constexpr double legendre01(int i, double t) { return
 // time), then the new ones; the projection runs after the Gauss loop in the order q. So
 // neither the previous coefficients nor the 30 projection sums are live while the point
 // arithmetic runs. Ocean and land elements take separate Gauss loops.
-// a0 + a1 X + a2 (X^2 - 1/12) at the Gauss points.
-template <int NG> __device__ __forceinline__ void legendreValues(double a0, double a1, double a2, double* v)
-{
-    const double g = gauss_point(NG, NG - 1) - 0.5;
-    if constexpr (NG == 3) {
-        const double e = a0 + (1.0 / 15.0) * a2;
-        v[0] = e - g * a1;
-        v[1] = a0 - (1.0 / 12.0) * a2;
-        v[2] = e + g * a1;
-    } else {
-        v[0] = a0 - g * a1; // two points: the quadratic vanishes there
-        v[1] = a0 + g * a1;
-    }
-}
-// at(q, value) for a DG field with coefficients c (degrees as in dgBasisAt).
-template <int DG, int NG, class AT> __device__ __forceinline__ void dgAtGauss(const double* c, const AT& at)
-{
-    const auto k = [&](int i) { return i < DG ? c[i < DG ? i : 0] : 0.0; };
-    double r0[NG], r1[NG], r2[NG], v[NG];
-    legendreValues<NG>(k(0), k(2), k(4), r0);
-    legendreValues<NG>(k(1), k(5), k(7), r1);
-    legendreValues<NG>(k(3), k(6), 0.0, r2);
-#pragma unroll
-    for (int gy = 0; gy < NG; ++gy) {
-        legendreValues<NG>(r0[gy], r1[gy], r2[gy], v);
-#pragma unroll
-        for (int gx = 0; gx < NG; ++gx)
-            at(gx + NG * gy, v[gx]);
-    }
-}
 // What the brittle update of an element reads besides its velocities: loaded at once, ahead
 // of the strain, so that one wait covers it (the loads return while the strain is formed).
 template <int CG, int DG> struct BrittleState {
@@ -3939,11 +3905,16 @@ template <int CG, int DG> struct DynImpl final : DynBase {
     {
         cg2dg.apply(mesh, brittle ? avgU.p : u.p, tr->velx(), brittle ? avgV.p : v.p, tr->vely(), s, prof);
         tr->reinitNormalVelocity();
-        double* t = budgetOn ? tally.p : nullptr;
-        tr->step(dt, A.p, t ? t + ne : nullptr);
-        tr->step(dt, h.p, t);
-        tr->limit(A.p, true, 1.0, true, 0.0, t ? t + 3 * ne : nullptr);
-        tr->limit(h.p, false, 0.0, true, 0.0, t ? t + 2 * ne : nullptr);
+        const Limits limA = Limits::both(1.0, 0.0), limH = Limits::min(0.0);
+        if (budgetOn) { // the limiters by themselves, with their change tallied
+            tr->step(dt, A.p, tally.p + ne);
+            tr->step(dt, h.p, tally.p);
+            tr->limit(A.p, limA, tally.p + 3 * ne);
+            tr->limit(h.p, limH, tally.p + 2 * ne);
+        } else {
+            tr->step(dt, A.p, nullptr, limA);
+            tr->step(dt, h.p, nullptr, limH);
+        }
     }
     void prepareIterationAsync()
     {
@@ -4425,8 +4396,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
         stressTr->reinitNormalVelocity();
         for (int c = 0; c < 3; ++c)
             stressTr->step(dt, sig.p + static_cast<size_t>(c) * S * ne);
-        tr->step(dt, damage.p);
-        tr->limit(damage.p, true, 1.0, true, 1e-12);
+        tr->step(dt, damage.p, nullptr, Limits::both(1.0, 1e-12));
         prepareIterationAsync();
         deltaT = dt / p.nsteps;
         deviceFill(avgU.p, nn, 0.0, s);

@@ -4,7 +4,8 @@
 // its cell term, the upwind fluxes of its four edges (each interior edge flux is
 // evaluated by both neighbours from identical operands, so the pair stays exactly
 // conservative without atomics), its Dirichlet outflow terms, the inverse mass
-// matrix and the Runge-Kutta stage combination, in one pass over HBM. Periodic
+// matrix and the Runge-Kutta stage combination (after the last stage of a step the
+// limiters too), in one pass over HBM. Periodic
 // segments, when present, are applied by a per-entry kernel between the flux pass
 // and a finishing pass. Fields are SoA (component-major) on the device.
 // Reference: dynamics/src/DGTransport.cpp:158-566, ParametricMap.cpp:13-87,
@@ -16,7 +17,7 @@
 
 namespace nsdg {
 
-enum StageMode { ST_RAW = 0, ST_PLUS = 1, ST_PLUS_K = 2, ST_RK2B = 3, ST_RK3B = 4, ST_RK3C = 5 };
+enum StageMode { ST_PLUS = 1, ST_RK2B = 3, ST_RK3B = 4, ST_RK3C = 5 };
 
 struct TrArgs {
     MeshView m;
@@ -30,51 +31,21 @@ struct TrArgs {
     size_t opStride;
     double dt;
     int mode;
-    const double* base; // RK3 base field (phi)
-    const double* kin;  // RK2 first-stage increment
-    double* kout;
+    const double* base; // the field the step starts from (RK2 and RK3 stages)
     double* out;
     double* raw;        // un-finished increment (periodic path)
     bool withDirichlet;
     double* tally;      // per-element Dirichlet outflow accumulator (mass budget), or null
     double tallyW;      // weight of this stage's outflow in the step (1/R folded in on the sphere)
+    Limits lim;         // limiters applied to the stage's result
 };
 
 // ---------------------------------------------------------------- operator set-up
-// AdvectionCellTermX/Y (ParametricMap.cpp:13-66) and the inverse DG mass matrix
-// (:68-87), k-major: cellX[i*Q+q], cellY[DG*Q + i*Q+q], invM[2*DG*Q + i*DG+j].
-template <int DG> __global__ void k_transport_ops(MeshView m, int nOps, double* ops)
-{
-    constexpr int G = gp1d(DG), Q = G * G;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nOps)
-        return;
-    double c[4][2];
-    elementCoords(m, e, c);
-    double dxT[2][Q], dyT[2][Q];
-    mapGradients<G>(c, dxT, dyT);
-    for (int i = 0; i < DG; ++i)
-        for (int q = 0; q < Q; ++q) {
-            const double w = W<G>::v[0][q];
-            const double X = Psi<DG, G>::x[i][q] * (dyT[1][q] * w) - Psi<DG, G>::y[i][q] * (dxT[1][q] * w);
-            const double Y = Psi<DG, G>::y[i][q] * (dxT[0][q] * w) - Psi<DG, G>::x[i][q] * (dyT[0][q] * w);
-            ops[static_cast<size_t>(i * Q + q) * nOps + e] = X;
-            ops[static_cast<size_t>(DG * Q + i * Q + q) * nOps + e] = Y;
-        }
-    // on the sphere: the cell terms stay the Cartesian ones in (longitude, latitude) and the
-    // inverse mass carries cos(latitude) and 1 / R (ParametricMap.cpp:49-80)
-    double M[DG][DG], Mi[DG][DG];
-    metricMassMatrix<DG>(m, c, M);
-    invert<DG>(M, Mi);
-    for (int i = 0; i < DG; ++i)
-        for (int j = 0; j < DG; ++j)
-            ops[static_cast<size_t>(2 * DG * Q + i * DG + j) * nOps + e]
-                = m.spherical ? Mi[i][j] / kEarthRadius : Mi[i][j];
-}
-
-// Transport operators of a general mesh from its geometry, SoA [k][ne]: the bilinear map
-// x(xi, eta) = x0 + X1 xi + X2 eta + X3 xi eta (and y), and the upper triangle of the
-// inverse (metric) DG mass matrix (/ R on the sphere). The cell terms factor through the map:
+// Transport operators from the mesh geometry, SoA [k][ne] (one element on a uniform mesh):
+// the bilinear map x(xi, eta) = x0 + X1 xi + X2 eta + X3 xi eta (and y), and the upper
+// triangle of the inverse (metric) DG mass matrix (/ R on the sphere; AdvectionCellTermX/Y
+// and the inverse mass, ParametricMap.cpp:13-87: on the sphere the cell terms stay the
+// Cartesian ones in (longitude, latitude)). The cell terms factor through the map:
 //   sum_q (cellX_i vx + cellY_i vy) phi = sum_q psi_xi,i (y_eta vx - x_eta vy) w phi
 //                                            + psi_eta,i (x_xi vy - y_xi vx) w phi,
 // so 6 + D (D + 1) / 2 values (27 for D = 6, 42 for D = 8) replace 2 D Q + D^2 (144, 208).
@@ -222,16 +193,10 @@ template <int DG> __device__ __forceinline__ void loadCell(const double* f, int 
     for (int i = 0; i < DG; ++i)
         c[i] = f[static_cast<size_t>(i) * ne + e];
 }
+// Edge coefficients (1, T, T^2 - 1/12) evaluated at the edge's Gauss points.
 template <int E, int G> __device__ __forceinline__ void edgeEval(const double* ev, double* out)
 {
-#pragma unroll
-    for (int q = 0; q < G; ++q) {
-        double s = 0;
-#pragma unroll
-        for (int k = 0; k < E; ++k)
-            s += ev[k] * PsiE<E, G>::v[k][q];
-        out[q] = s;
-    }
+    legendreValues<G>(ev[0], E > 1 ? ev[E > 1 ? 1 : 0] : 0.0, E > 2 ? ev[E > 2 ? 2 : 0] : 0.0, out);
 }
 template <int E> __device__ __forceinline__ void loadEdge(const double* nv, int n, int ie, double* v)
 {
@@ -239,23 +204,49 @@ template <int E> __device__ __forceinline__ void loadEdge(const double* nv, int 
     for (int k = 0; k < E; ++k)
         v[k] = nv[static_cast<size_t>(k) * n + ie];
 }
-// up += sgn * sum_q dt * tmp[q] * PSIe_w<side>[q][i]
+// Moments of edge values against (1, T, T^2 - 1/12) under the Gauss rule.
+template <int E, int G> __device__ __forceinline__ void edgeMoments(const double* f, double* m)
+{
+    const double g = gauss_point(G, G - 1) - 0.5;
+    if constexpr (G == 1) {
+        m[0] = f[0];
+    } else if constexpr (G == 2) {
+        m[0] = 0.5 * (f[0] + f[1]);
+        m[1] = (0.5 * g) * (f[1] - f[0]);
+    } else {
+        const double a = f[0] + f[2];
+        m[0] = (5.0 / 18.0) * a + (8.0 / 18.0) * f[1];
+        m[1] = (5.0 / 18.0 * g) * (f[2] - f[0]);
+        m[2] = (1.0 / 54.0) * a - (1.0 / 27.0) * f[1];
+    }
+}
+// up += sgn * dt * sum_q tmp[q] w_q PSI(side, q): the transpose of the trace, from the edge
+// moments.
 template <int DG, int SIDE>
 __device__ __forceinline__ void edgeAccumulate(double* up, double sgn, double dt, const double* tmp)
 {
-    constexpr int G = gp1d(DG);
+    constexpr int E = edgedofs(DG), G = gp1d(DG);
+    constexpr double s = (SIDE == 0 || SIDE == 3) ? -0.5 : 0.5;
+    constexpr bool X = SIDE == 1 || SIDE == 3; // x~ = s along the edge, else y~ = s
+    double m[E];
+    edgeMoments<E, G>(tmp, m);
+    const double f = sgn * dt;
 #pragma unroll
-    for (int i = 0; i < DG; ++i) {
-        double s = 0;
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-            const double w = SIDE == 0 ? PsiEW<DG, G>::b[q][i]
-                : SIDE == 1            ? PsiEW<DG, G>::r[q][i]
-                : SIDE == 2            ? PsiEW<DG, G>::t[q][i]
-                                       : PsiEW<DG, G>::l[q][i];
-            s += dt * tmp[q] * w;
-        }
-        up[i] += sgn * s;
+    for (int k = 0; k < E; ++k)
+        m[k] *= f;
+    up[0] += m[0];
+    if constexpr (DG > 1) {
+        up[X ? 1 : 2] += s * m[0];
+        up[X ? 2 : 1] += m[1];
+    }
+    if constexpr (DG > 3) {
+        up[X ? 3 : 4] += (1.0 / 6.0) * m[0];
+        up[X ? 4 : 3] += m[2];
+        up[5] += s * m[1];
+    }
+    if constexpr (DG > 6) {
+        up[X ? 6 : 7] += (1.0 / 6.0) * m[1];
+        up[X ? 7 : 6] += s * m[2];
     }
 }
 // Upwind flux through an interior edge between c1 (left/bottom, side S1 of c1) and
@@ -291,16 +282,9 @@ __device__ __forceinline__ double boundaryTerm(double* up, const double* ph, con
         tmp[q] = pg[q] * fmax(sgn * vg[q], 0.0);
     for (int r = 0; r < count; ++r)
         edgeAccumulate<DG, SIDE>(up, -1.0, dt, tmp);
-    double o = 0;
-#pragma unroll
-    for (int q = 0; q < G; ++q) {
-        const double w = SIDE == 0 ? PsiEW<DG, G>::b[q][0]
-            : SIDE == 1            ? PsiEW<DG, G>::r[q][0]
-            : SIDE == 2            ? PsiEW<DG, G>::t[q][0]
-                                   : PsiEW<DG, G>::l[q][0];
-        o += dt * tmp[q] * w;
-    }
-    return count * o;
+    double m[E];
+    edgeMoments<E, G>(tmp, m);
+    return count * (dt * m[0]);
 }
 // All Dirichlet terms of element e; with a.tally set, the stage-weighted outflow is added
 // to the element's budget accumulator (elements without Dirichlet sides add nothing).
@@ -331,37 +315,91 @@ template <int DG> __device__ __forceinline__ void dirichletTerms(const TrArgs& a
     if (a.tally)
         a.tally[e] += a.tallyW * out;
 }
-// Inverse mass matrix and Runge-Kutta stage combination (DGTransport.cpp:509-552).
-template <int DG, bool UNI> __device__ __forceinline__ void finishCell(const TrArgs& a, int e, const double* ph, const double* up)
+// LimitMax then LimitMin (dgLimit.hpp:16-84) of one cell.
+template <int DG> __device__ __forceinline__ void limitCell(const Limits& l, double* c)
 {
-    constexpr int Q = gp1d(DG) * gp1d(DG);
-    const Ops<UNI> op { a.ops, a.opStride };
-    const size_t ne = a.ne;
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+        const bool isMax = pass == 0;
+        if (isMax ? !l.doMax : !l.doMin)
+            continue;
+        const double b = isMax ? l.maxv : l.minv;
+        c[0] = isMax ? fmin(b, c[0]) : fmax(b, c[0]);
+        if constexpr (DG == 3) {
+            const double l0 = 2.0 * fmax(fabs(c[1] + c[2]), fabs(c[1] - c[2]));
+            if (l0 != 0.0) {
+                const bool ex = isMax ? (c[0] + l0 - b > 0) : (c[0] - l0 - b < 0);
+                if (ex) {
+                    const double s = isMax ? (b - c[0]) / l0 : (c[0] - b) / l0;
+                    c[1] *= s;
+                    c[2] *= s;
+                }
+            }
+        } else if constexpr (DG == 6) {
+            double ext = isMax ? -INFINITY : INFINITY;
+            dgAtGauss<6, 3>(c, [&](int, double v) { ext = isMax ? fmax(ext, v) : fmin(ext, v); });
+            const double l0 = ext - c[0];
+            if (isMax ? (ext > b) : (ext < b)) {
+                const double s = isMax ? (b - c[0]) / l0 : (c[0] - b) / l0;
+#pragma unroll
+                for (int k = 1; k < 6; ++k)
+                    c[k] *= s;
+            }
+        }
+    }
+}
+// The inverse mass of element e (its upper triangle row by row; an affine element's is
+// diagonal).
+template <int DG, bool UNI> struct InverseMass {
+    static constexpr int K = UNI ? 1 : DG * (DG + 1) / 2;
+    double m[K];
+    __device__ __forceinline__ void load(const double* ops, size_t ne, int e)
+    {
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            m[k] = UNI ? ops[TrGeo<DG>::MI] : ops[(TrGeo<DG>::MI + k) * ne + e];
+    }
+    __device__ __forceinline__ void apply(const double* up, double* k) const
+    {
+        if constexpr (UNI) {
+#pragma unroll
+            for (int i = 0; i < DG; ++i)
+                k[i] = (m[0] * invMassRef(i)) * up[i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < DG; ++i)
+                k[i] = 0.0;
+            int n = 0;
+#pragma unroll
+            for (int i = 0; i < DG; ++i)
+#pragma unroll
+                for (int j = i; j < DG; ++j, ++n) {
+                    k[i] += m[n] * up[j];
+                    if (j != i)
+                        k[j] += m[n] * up[i];
+                }
+        }
+    }
+};
+// The Runge-Kutta stage combination (DGTransport.cpp:509-552) from the cell's operator input
+// ph, its increment k and the step's base field, then the limiters.
+template <int DG> __device__ __forceinline__ void finishCell(const TrArgs& a, int e, const double* ph, const double* k,
+    const double* base)
+{
+    double r[DG];
 #pragma unroll
     for (int i = 0; i < DG; ++i) {
-        double k = 0;
-#pragma unroll
-        for (int j = 0; j < DG; ++j) {
-            if constexpr (UNI)
-                k += op(2 * DG * Q + i * DG + j, e) * up[j];
-            else
-                k += a.ops[static_cast<size_t>(TrGeo<DG>::mi(i, j)) * ne + e] * up[j];
-        }
-        const size_t o = i * ne + e;
-        double r;
         switch (a.mode) {
-        case ST_RAW: r = k; break;
-        case ST_PLUS: r = ph[i] + k; break;
-        case ST_PLUS_K:
-            a.kout[o] = k;
-            r = ph[i] + k;
-            break;
-        case ST_RK2B: r = ph[i] + 0.5 * (k - a.kin[o]); break;
-        case ST_RK3B: r = (k + ph[i]) * 0.25 + 0.75 * a.base[o]; break;
-        default: r = a.base[o] * (1.0 / 3.0) + 2.0 / 3.0 * (k + ph[i]); break;
+        case ST_PLUS: r[i] = ph[i] + k[i]; break;
+        case ST_RK2B: r[i] = 0.5 * (base[i] + (ph[i] + k[i])); break; // phi + (k1 + k2) / 2, ph = phi + k1
+        case ST_RK3B: r[i] = (k[i] + ph[i]) * 0.25 + 0.75 * base[i]; break;
+        default: r[i] = base[i] * (1.0 / 3.0) + 2.0 / 3.0 * (k[i] + ph[i]); break;
         }
-        a.out[o] = r;
     }
+    limitCell<DG>(a.lim, r);
+#pragma unroll
+    for (int i = 0; i < DG; ++i)
+        a.out[static_cast<size_t>(i) * a.ne + e] = r[i];
 }
 
 // ---------------------------------------------------------------- DGTransportOperator
@@ -370,6 +408,13 @@ template <int DG, bool UNI> __device__ __forceinline__ void finishCell(const TrA
 // One element per thread; the runs of kBlock elements go to the XCDs in contiguous chunks
 // (xcdTile), so the rows above and below a run, which its edge fluxes read, were loaded
 // into the same XCD's L2 by the neighbouring runs.
+// Bound by the latency of its loads and by its traffic. Every load is issued at the start, in
+// the order of its use and whatever the ocean flags say (a clamped neighbour where there is
+// none), instead of behind the flag of each neighbour; values and moments at the Gauss
+// points go through the factors of the basis; an affine element's inverse mass is diagonal.
+// Per stage: 500 x 333 non-affine, D = 6, 24.8 -> 15.8 us with the limiters in the last stage
+// (4.8 us as a kernel of their own); 512 x 512 uniform 22.0 -> 15.5 us, D = 8 25.8 -> 18.8;
+// 2048 x 2048 336 -> 260 us.
 template <int DG, bool UNI, bool FINISH> __global__ __launch_bounds__(kBlock) void k_transport_op(TrArgs a)
 {
     constexpr int G = gp1d(DG), Q = G * G, E = edgedofs(DG);
@@ -379,94 +424,116 @@ template <int DG, bool UNI, bool FINISH> __global__ __launch_bounds__(kBlock) vo
     const int e = run * kBlock + threadIdx.x;
     if (e >= a.ne)
         return;
-    const int nx = a.m.nx, ny = a.m.ny, ix = e % nx, iy = e / nx, ne = a.ne;
-    const Ops<UNI> op { a.ops, a.opStride };
-    double ph[DG], up[DG];
-    loadCell<DG>(a.x, ne, e, ph);
+    const int nx = a.m.nx, ny = a.m.ny, ix = e % nx, iy = e / nx;
+    const size_t ne = a.ne;
+    // left, right, bottom, top: the neighbour and the edge
+    const int nbr[4] = { ix > 0 ? e - 1 : e, ix < nx - 1 ? e + 1 : e, iy > 0 ? e - nx : e, iy < ny - 1 ? e + nx : e };
+    const int edge[4] = { iy * (nx + 1) + ix, iy * (nx + 1) + ix + 1, ix + nx * iy, ix + nx * (iy + 1) };
+    const bool oc = a.m.ocean[e] != 0;
+    bool has[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+        has[s] = a.m.ocean[nbr[s]] != 0;
+    double ph[DG], up[DG], vx[DG], vy[DG], nb[4][DG], nv[4][E], base[DG], map[6];
+    loadCell<DG>(a.x, a.ne, e, ph);
+    if constexpr (DG > 1) {
+        loadCell<DG>(a.velx, a.ne, e, vx);
+        loadCell<DG>(a.vely, a.ne, e, vy);
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+            map[k] = UNI ? a.ops[k] : a.ops[k * ne + e];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        loadCell<DG>(a.x, a.ne, nbr[s], nb[s]);
+        loadEdge<E>(s < 2 ? a.nvY : a.nvX, s < 2 ? a.nYe : a.nXe, edge[s], nv[s]);
+    }
+    // the 36 values of D = 8 would not fit in registers as early
+    constexpr bool kEarly = UNI || DG < 8;
+    InverseMass<DG, UNI> im;
+    if constexpr (FINISH) {
+        if (kEarly)
+            im.load(a.ops, ne, e);
+        if (a.base)
+            loadCell<DG>(a.base, a.ne, e, base);
+    }
+    has[0] = has[0] && oc && ix > 0;
+    has[1] = has[1] && oc && ix < nx - 1;
+    has[2] = has[2] && oc && iy > 0;
+    has[3] = has[3] && oc && iy < ny - 1;
 #pragma unroll
     for (int i = 0; i < DG; ++i)
         up[i] = 0.0;
-    const bool oc = a.m.ocean[e];
     if constexpr (DG > 1) {
-        if (oc) { // cell_term (DGTransport.cpp:278-303)
-            double vx[DG], vy[DG], vxg[Q], vyg[Q], pg[Q];
-            loadCell<DG>(a.velx, ne, e, vx);
-            loadCell<DG>(a.vely, ne, e, vy);
+        if (oc) {
+            // cell_term (DGTransport.cpp:278-303): the fluxes phi (y_eta vx - x_eta vy) w and
+            // phi (x_xi vy - y_xi vx) w against psi_xi and psi_eta
+            double vxg[Q], vyg[Q], F[Q], H[Q];
+            dgAtGauss<DG, G>(vx, [&](int q, double v) { vxg[q] = v; });
+            dgAtGauss<DG, G>(vy, [&](int q, double v) { vyg[q] = v; });
+            dgAtGauss<DG, G>(ph, [&](int q, double v) {
+                const double xi = gauss_point(G, q % G), eta = gauss_point(G, q / G);
+                const double w = (gauss_weight(G, q % G) * gauss_weight(G, q / G)) * v * a.dt;
+                const double xxi = UNI ? map[0] : map[0] + map[2] * eta, xeta = UNI ? map[1] : map[1] + map[2] * xi;
+                const double yxi = UNI ? map[3] : map[3] + map[5] * eta, yeta = UNI ? map[4] : map[4] + map[5] * xi;
+                F[q] = (yeta * vxg[q] - xeta * vyg[q]) * w;
+                H[q] = (xxi * vyg[q] - yxi * vxg[q]) * w;
+            });
+            if constexpr (G == 3) {
+                const double g = gauss_point(3, 2) - 0.5;
+                double s[3], d[3], p[3], t[3];
 #pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                double s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-                for (int i = 0; i < DG; ++i) {
-                    s0 += vx[i] * Psi<DG, G>::v[i][q];
-                    s1 += vy[i] * Psi<DG, G>::v[i][q];
-                    s2 += ph[i] * Psi<DG, G>::v[i][q];
+                for (int y = 0; y < 3; ++y) {
+                    s[y] = F[3 * y] + F[3 * y + 1] + F[3 * y + 2];
+                    d[y] = F[3 * y + 2] - F[3 * y];     // X moment / g
+                    p[y] = H[y] + H[y + 3] + H[y + 6];  // by column
+                    t[y] = H[y + 6] - H[y];             // Y moment / g
                 }
-                vxg[q] = s0;
-                vyg[q] = s1;
-                pg[q] = s2;
-            }
-            if constexpr (UNI) {
-#pragma unroll
-                for (int i = 0; i < DG; ++i) {
-                    double s = 0;
-#pragma unroll
-                    for (int q = 0; q < Q; ++q)
-                        s += a.dt * (op(i * Q + q, e) * vxg[q] + op(DG * Q + i * Q + q, e) * vyg[q]) * pg[q];
-                    up[i] += s;
+                up[1] = s[0] + s[1] + s[2];
+                up[2] = p[0] + p[1] + p[2];
+                up[3] = (2.0 * g) * (d[0] + d[1] + d[2]);
+                up[4] = (2.0 * g) * (t[0] + t[1] + t[2]);
+                up[5] = g * ((s[2] - s[0]) + (p[2] - p[0]));
+                if constexpr (DG == 8) {
+                    up[6] = (2.0 * g * g) * (d[2] - d[0]) + ((1.0 / 15.0) * (p[0] + p[2]) - (1.0 / 12.0) * p[1]);
+                    up[7] = (2.0 * g * g) * (t[2] - t[0]) + ((1.0 / 15.0) * (s[0] + s[2]) - (1.0 / 12.0) * s[1]);
                 }
             } else {
-                using L = TrGeo<DG>;
-                const size_t sne = static_cast<size_t>(ne);
-                const double X1 = a.ops[L::X1 * sne + e], X2 = a.ops[L::X2 * sne + e], X3 = a.ops[L::X3 * sne + e];
-                const double Y1 = a.ops[L::Y1 * sne + e], Y2 = a.ops[L::Y2 * sne + e], Y3 = a.ops[L::Y3 * sne + e];
-#pragma unroll
-                for (int q = 0; q < Q; ++q) {
-                    const double xi = gauss_point(G, q % G), eta = gauss_point(G, q / G);
-                    const double w = gauss_weight(G, q % G) * gauss_weight(G, q / G) * a.dt;
-                    const double xxi = X1 + X3 * eta, xeta = X2 + X3 * xi, yxi = Y1 + Y3 * eta, yeta = Y2 + Y3 * xi;
-                    const double fxi = (yeta * vxg[q] - xeta * vyg[q]) * (w * pg[q]);
-                    const double feta = (xxi * vyg[q] - yxi * vxg[q]) * (w * pg[q]);
-#pragma unroll
-                    for (int i = 0; i < DG; ++i)
-                        up[i] += Psi<DG, G>::x[i][q] * fxi + Psi<DG, G>::y[i][q] * feta;
-                }
+                up[1] = (F[0] + F[1]) + (F[2] + F[3]);
+                up[2] = (H[0] + H[1]) + (H[2] + H[3]);
             }
         }
     }
-    if (oc) {
-        double nb[DG], nv[E], tmp[G];
-        if (ix > 0 && a.m.ocean[e - 1]) { // left Y-edge: this cell is c2
-            loadCell<DG>(a.x, ne, e - 1, nb);
-            loadEdge<E>(a.nvY, a.nYe, iy * (nx + 1) + ix, nv);
-            upwind<DG, 1, 3>(nb, ph, nv, tmp);
-            edgeAccumulate<DG, 3>(up, 1.0, a.dt, tmp);
-        }
-        if (ix < nx - 1 && a.m.ocean[e + 1]) { // right Y-edge: this cell is c1
-            loadCell<DG>(a.x, ne, e + 1, nb);
-            loadEdge<E>(a.nvY, a.nYe, iy * (nx + 1) + ix + 1, nv);
-            upwind<DG, 1, 3>(ph, nb, nv, tmp);
-            edgeAccumulate<DG, 1>(up, -1.0, a.dt, tmp);
-        }
-        if (iy > 0 && a.m.ocean[e - nx]) { // bottom X-edge: this cell is c2
-            loadCell<DG>(a.x, ne, e - nx, nb);
-            loadEdge<E>(a.nvX, a.nXe, ix + nx * iy, nv);
-            upwind<DG, 2, 0>(nb, ph, nv, tmp);
-            edgeAccumulate<DG, 0>(up, 1.0, a.dt, tmp);
-        }
-        if (iy < ny - 1 && a.m.ocean[e + nx]) { // top X-edge: this cell is c1
-            loadCell<DG>(a.x, ne, e + nx, nb);
-            loadEdge<E>(a.nvX, a.nXe, ix + nx * (iy + 1), nv);
-            upwind<DG, 2, 0>(ph, nb, nv, tmp);
-            edgeAccumulate<DG, 2>(up, -1.0, a.dt, tmp);
-        }
-    }
+    // edge fluxes: this cell is c2 of its left and bottom edges, c1 of the others
+    double tmp[G];
+    const auto masked = [&](bool h) {
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+            tmp[q] = h ? tmp[q] : 0.0;
+    };
+    upwind<DG, 1, 3>(nb[0], ph, nv[0], tmp);
+    masked(has[0]);
+    edgeAccumulate<DG, 3>(up, 1.0, a.dt, tmp);
+    upwind<DG, 1, 3>(ph, nb[1], nv[1], tmp);
+    masked(has[1]);
+    edgeAccumulate<DG, 1>(up, -1.0, a.dt, tmp);
+    upwind<DG, 2, 0>(nb[2], ph, nv[2], tmp);
+    masked(has[2]);
+    edgeAccumulate<DG, 0>(up, 1.0, a.dt, tmp);
+    upwind<DG, 2, 0>(ph, nb[3], nv[3], tmp);
+    masked(has[3]);
+    edgeAccumulate<DG, 2>(up, -1.0, a.dt, tmp);
     if constexpr (FINISH) {
         dirichletTerms<DG>(a, e, ph, up);
-        finishCell<DG, UNI>(a, e, ph, up);
+        double k[DG];
+        if (!kEarly)
+            im.load(a.ops, ne, e);
+        im.apply(up, k);
+        finishCell<DG>(a, e, ph, k, base);
     } else {
 #pragma unroll
         for (int i = 0; i < DG; ++i)
-            a.raw[static_cast<size_t>(i) * ne + e] = up[i];
+            a.raw[i * ne + e] = up[i];
     }
 }
 
@@ -508,19 +575,23 @@ template <int DG, bool UNI> __global__ __launch_bounds__(kBlock) void k_transpor
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= a.ne)
         return;
-    double ph[DG], up[DG];
+    double ph[DG], up[DG], base[DG], k[DG];
     loadCell<DG>(a.x, a.ne, e, ph);
     loadCell<DG>(a.raw, a.ne, e, up);
+    if (a.base)
+        loadCell<DG>(a.base, a.ne, e, base);
+    InverseMass<DG, UNI> im;
+    im.load(a.ops, a.ne, e);
     dirichletTerms<DG>(a, e, ph, up);
-    finishCell<DG, UNI>(a, e, ph, up);
+    im.apply(up, k);
+    finishCell<DG>(a, e, ph, k, base);
 }
 
 // ---------------------------------------------------------------- limiters
-// LimitMax then LimitMin (dgLimit.hpp:16-84) on one SoA field. With tally set, the change
+// The limiters on one SoA field by themselves. With tally set, the change
 // of the element's Tools::MeanValue contribution is added to tally[e] (mass budget).
 template <int DG>
-__global__ void k_limit(MeshView m, double* f, int ne, bool doMax, double maxv, bool doMin, double minv,
-    double* tally)
+__global__ __launch_bounds__(kBlock) void k_limit(MeshView m, double* f, int ne, Limits lim, double* tally)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= ne)
@@ -530,41 +601,7 @@ __global__ void k_limit(MeshView m, double* f, int ne, bool doMax, double maxv, 
 #pragma unroll
     for (int i = 0; i < DG; ++i)
         c0[i] = c[i];
-    for (int pass = 0; pass < 2; ++pass) {
-        const bool isMax = pass == 0;
-        if (isMax ? !doMax : !doMin)
-            continue;
-        const double b = isMax ? maxv : minv;
-        c[0] = isMax ? fmin(b, c[0]) : fmax(b, c[0]);
-        if constexpr (DG == 3) {
-            const double l0 = 2.0 * fmax(fabs(c[1] + c[2]), fabs(c[1] - c[2]));
-            if (l0 != 0.0) {
-                const bool ex = isMax ? (c[0] + l0 - b > 0) : (c[0] - l0 - b < 0);
-                if (ex) {
-                    const double s = isMax ? (b - c[0]) / l0 : (c[0] - b) / l0;
-                    c[1] *= s;
-                    c[2] *= s;
-                }
-            }
-        } else if constexpr (DG == 6) {
-            double ext = isMax ? -INFINITY : INFINITY;
-#pragma unroll
-            for (int q = 0; q < 9; ++q) {
-                double s = 0;
-#pragma unroll
-                for (int k = 0; k < 6; ++k)
-                    s += c[k] * Psi<6, 3>::v[k][q];
-                ext = isMax ? fmax(ext, s) : fmin(ext, s);
-            }
-            const double l0 = ext - c[0];
-            if (isMax ? (ext > b) : (ext < b)) {
-                const double s = isMax ? (b - c[0]) / l0 : (c[0] - b) / l0;
-#pragma unroll
-                for (int k = 1; k < 6; ++k)
-                    c[k] *= s;
-            }
-        }
-    }
+    limitCell<DG>(lim, c);
     // a cell the limits leave bit for bit as it was is not written back (most cells)
     bool moved = false;
 #pragma unroll
@@ -786,7 +823,7 @@ template <int DG> struct TransportImpl final : TransportBase {
     Profiler& prof;
     int scheme = 2;
     int nXe, nYe;
-    DBuf<double> ops, vx, vy, nvX, nvY, tmpA, tmpB, kbuf, raw, scratch;
+    DBuf<double> ops, vx, vy, nvX, nvY, tmpA, tmpB, raw, scratch;
     CG2DGOps cg2dg[3];
 
     TransportImpl(DeviceMesh& m, hipStream_t st, Profiler& p)
@@ -797,15 +834,11 @@ template <int DG> struct TransportImpl final : TransportBase {
         const size_t ne = mesh.ne;
         nXe = mesh.nx * (mesh.ny + 1);
         nYe = (mesh.nx + 1) * mesh.ny;
-        if (mesh.uniform) {
-            ops.alloc(static_cast<size_t>(2 * DG * Q + DG * DG));
-            k_transport_ops<DG><<<1, kBlock, 0, s>>>(view(mesh), 1, ops.p);
-        } else {
-            ops.alloc(static_cast<size_t>(TrGeo<DG>::K) * ne);
-            k_transport_geom<DG><<<blocksFor(ne), kBlock, 0, s>>>(view(mesh), static_cast<int>(ne), ops.p);
-        }
+        const size_t nOps = mesh.uniform ? 1 : ne;
+        ops.alloc(static_cast<size_t>(TrGeo<DG>::K) * nOps);
+        k_transport_geom<DG><<<blocksFor(nOps), kBlock, 0, s>>>(view(mesh), static_cast<int>(nOps), ops.p);
         checkLaunch("transport_ops");
-        for (auto* b : { &vx, &vy, &tmpA, &tmpB, &kbuf, &raw })
+        for (auto* b : { &vx, &vy, &tmpA, &tmpB, &raw })
             b->alloc(ne * DG);
         nvX.alloc(static_cast<size_t>(E) * nXe);
         nvY.alloc(static_cast<size_t>(E) * nYe);
@@ -902,8 +935,9 @@ template <int DG> struct TransportImpl final : TransportBase {
     }
     // step_rk1 / step_rk2 / step_rk3 (DGTransport.cpp:514-552) on a device field. With
     // tally set, each element's Dirichlet outflow over the step (in MeanValue units) is
-    // added to tally[e]: the stage outflows weighted as the stages enter the new field.
-    void step(double dt, double* phi, double* tally) override
+    // added to tally[e]: the stage outflows weighted as the stages enter the new field. The
+    // limiters lim are applied to the new field in its last stage.
+    void step(double dt, double* phi, double* tally, const Limits& lim) override
     {
         const size_t n = mesh.ne * DG;
         // on the sphere the inverse mass carries 1/R (ParametricMap.cpp:68-87)
@@ -917,18 +951,19 @@ template <int DG> struct TransportImpl final : TransportBase {
             TrArgs a = withTally(args(dt, phi), 1.0);
             a.mode = ST_PLUS;
             a.out = tmpA.p;
+            a.lim = lim;
             stage(a);
             deviceCopy(phi, tmpA.p, n, s);
         } else if (scheme == 2) { // phi + (k1 + k2) / 2
             TrArgs a = withTally(args(dt, phi), 0.5);
-            a.mode = ST_PLUS_K;
-            a.kout = kbuf.p;
+            a.mode = ST_PLUS;
             a.out = tmpA.p;
             stage(a);
             TrArgs b = withTally(args(dt, tmpA.p), 0.5);
             b.mode = ST_RK2B;
-            b.kin = kbuf.p;
+            b.base = phi;
             b.out = phi;
+            b.lim = lim;
             stage(b);
         } else { // phi + (k1 + k2) / 6 + 2 k3 / 3
             TrArgs a = withTally(args(dt, phi), 1.0 / 6.0);
@@ -944,14 +979,14 @@ template <int DG> struct TransportImpl final : TransportBase {
             c.mode = ST_RK3C;
             c.base = phi;
             c.out = phi;
+            c.lim = lim;
             stage(c);
         }
     }
-    void limit(double* phi, bool doMax, double maxv, bool doMin, double minv, double* tally) override
+    void limit(double* phi, const Limits& lim, double* tally) override
     {
         Timed t(prof, s, "limit");
-        k_limit<DG><<<blocksFor(mesh.ne), kBlock, 0, s>>>(
-            view(mesh), phi, static_cast<int>(mesh.ne), doMax, maxv, doMin, minv, tally);
+        k_limit<DG><<<blocksFor(mesh.ne), kBlock, 0, s>>>(view(mesh), phi, static_cast<int>(mesh.ne), lim, tally);
         checkLaunch("limit");
     }
 };

@@ -6,6 +6,15 @@
 
 namespace nsdg {
 
+// LimitMax(field, maxv) and LimitMin(field, minv) (dgLimit.hpp:16-84), in that order.
+struct Limits {
+    bool doMax = false, doMin = false;
+    double maxv = 0, minv = 0;
+    static Limits max(double v) { return { true, false, v, 0 }; }
+    static Limits min(double v) { return { false, true, 0, v }; }
+    static Limits both(double hi, double lo) { return { true, true, hi, lo }; }
+};
+
 // Runtime-degree interface over TransportImpl<DG>.
 struct TransportBase {
     virtual ~TransportBase() = default;
@@ -15,10 +24,10 @@ struct TransportBase {
     virtual void prepareAdvectionHost(int cg, const double* u, const double* v) = 0;
     virtual void reinitNormalVelocity() = 0;
     // SoA field on the device; tally (optional, N_e doubles) accumulates each element's
-    // Dirichlet outflow in Tools::MeanValue units
-    virtual void step(double dt, double* phiDev, double* tally = nullptr) = 0;
+    // Dirichlet outflow in Tools::MeanValue units; lim is applied to the new field
+    virtual void step(double dt, double* phiDev, double* tally = nullptr, const Limits& lim = {}) = 0;
     // tally (optional) accumulates the change of each element's MeanValue contribution
-    virtual void limit(double* phiDev, bool doMax, double maxv, bool doMin, double minv, double* tally = nullptr) = 0;
+    virtual void limit(double* phiDev, const Limits& lim, double* tally = nullptr) = 0;
     virtual double* velx() = 0;
     virtual double* vely() = 0;
 };
