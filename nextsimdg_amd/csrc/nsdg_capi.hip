@@ -201,8 +201,7 @@ int nsdg_transport_run(nsdg_transport* t, double dt, double* phi, int nsteps, in
         require(nsteps >= 0, "nsteps must be >= 0");
         auto& h = t->h;
         const int dg = h.t->dg();
-        DBuf<double> scratch;
-        uploadSoA(scratch, phi, h.mesh.ne, dg, h.field.p, h.stream);
+        uploadSoA(h.io, phi, h.mesh.ne, dg, h.field.p, h.stream);
         // the steps do not change the velocity: its normal components once for all of them
         // (500 x 333, D = 6: 13.8 us of each step's 68)
         if (nsteps > 0)
@@ -210,7 +209,7 @@ int nsdg_transport_run(nsdg_transport* t, double dt, double* phi, int nsteps, in
         const Limits lim { (limit_flags & 1) != 0, (limit_flags & 2) != 0, 1.0, 0.0 };
         for (int k = 0; k < nsteps; ++k)
             h.t->step(dt, h.field.p, nullptr, lim);
-        downloadSoA(scratch, h.field.p, h.mesh.ne, dg, phi, h.stream);
+        downloadSoA(h.io, h.field.p, h.mesh.ne, dg, phi, h.stream);
     });
 }
 int nsdg_transport_step(nsdg_transport* t, double dt, double* phi)
@@ -220,10 +219,9 @@ int nsdg_transport_step(nsdg_transport* t, double dt, double* phi)
         nonNull(phi, "phi");
         auto& h = t->h;
         const int dg = h.t->dg();
-        DBuf<double> scratch;
-        uploadSoA(scratch, phi, h.mesh.ne, dg, h.field.p, h.stream);
+        uploadSoA(h.io, phi, h.mesh.ne, dg, h.field.p, h.stream);
         h.t->step(dt, h.field.p);
-        downloadSoA(scratch, h.field.p, h.mesh.ne, dg, phi, h.stream);
+        downloadSoA(h.io, h.field.p, h.mesh.ne, dg, phi, h.stream);
     });
 }
 int nsdg_transport_destroy(nsdg_transport* t)
@@ -253,14 +251,14 @@ int nsdg_limit(int dg, size_t n, double* phi, double bound, int is_max)
         m.create(nxm, 2, coords.data());
         h.mesh.build(m, h.stream);
         h.t = makeTransport(dg, h.mesh, h.stream, h.prof);
-        DBuf<double> f, scratch;
+        DBuf<double> f;
         f.alloc(h.mesh.ne * dg);
         deviceFill(f.p, f.n, 0.0, h.stream);
         std::vector<double> full(h.mesh.ne * dg, 0.0);
         std::memcpy(full.data(), phi, n * dg * sizeof(double));
-        uploadSoA(scratch, full.data(), h.mesh.ne, dg, f.p, h.stream);
+        uploadSoA(h.io, full.data(), h.mesh.ne, dg, f.p, h.stream);
         h.t->limit(f.p, is_max != 0 ? Limits::max(bound) : Limits::min(bound));
-        downloadSoA(scratch, f.p, h.mesh.ne, dg, full.data(), h.stream);
+        downloadSoA(h.io, f.p, h.mesh.ne, dg, full.data(), h.stream);
         std::memcpy(phi, full.data(), n * dg * sizeof(double));
     });
 }

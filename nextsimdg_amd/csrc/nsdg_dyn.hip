@@ -3543,7 +3543,8 @@ template <int CG, int DG> struct DynImpl final : DynBase {
     double deltaT = 0;
     DBuf<double> mops, geo, brittleGeo, lumped, lumped1, h, A, ssh, eps, sig;
     DBuf<double> u, v, u0, v0, uo, vo, ua, va, cgH, cgA, gX, gY, dSx, dSy;
-    DBuf<double> tmpDG, tmpDG2, tmpCG, tmpCG2, cg1a, cg1b, cg1c, scratch, dg0a, dg0b, part, res;
+    DBuf<double> tmpDG, tmpDG2, tmpCG, tmpCG2, cg1a, cg1b, cg1c, dg0a, dg0b, part, res;
+    HostIO io;
     DBuf<uint8_t> dirNode;
     DBuf<double2> fzOcn, fzCf, fzQ; // frozen momentum coefficients (k_node_coeffs)
     DBuf<double> strength;          // ice strength at the Gauss points
@@ -3785,7 +3786,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
     void dg0ToCG(const double* data, int ncomp, double* dst)
     {
         if (ncomp == DG) {
-            uploadSoA(scratch, data, ne, DG, tmpDG.p, s);
+            uploadSoA(io, data, ne, DG, tmpDG.p, s);
             launchDG2CG<DG>(tmpDG.p, dst, 0, nullptr, nullptr, 0);
         } else {
             require(ncomp == 1, "field must have 1 or DG components");
@@ -3813,7 +3814,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
             double* f = n == "hice" ? h.p : (n == "cice" ? A.p : damage.p);
             require(ncomp == 1 || ncomp == DG, "hice/cice/damage need 1 or DG components");
             if (ncomp == DG)
-                uploadSoA(scratch, data, ne, DG, f, s);
+                uploadSoA(io, data, ne, DG, f, s);
             else {
                 deviceFill(f, ne * DG, 0.0, s);
                 NSDG_HIP(hipMemcpyAsync(f, data, ne * sizeof(double), hipMemcpyHostToDevice, s));
@@ -3824,7 +3825,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
         } else if (double* t = tensorRef(n)) {
             require(ncomp == 1 || ncomp == S, "stress/strain need 1 or S components");
             if (ncomp == S)
-                uploadSoA(scratch, data, ne, S, t, s);
+                uploadSoA(io, data, ne, S, t, s);
             else {
                 deviceFill(t, ne * S, 0.0, s);
                 NSDG_HIP(hipMemcpyAsync(t, data, ne * sizeof(double), hipMemcpyHostToDevice, s));
@@ -3854,16 +3855,16 @@ template <int CG, int DG> struct DynImpl final : DynBase {
                 src = n == "uiostress" ? tmpCG.p : tmpCG2.p;
             }
             cg2dg.apply(mesh, src, tmpDG.p, nullptr, nullptr, s, prof);
-            downloadSoA(scratch, tmpDG.p, ne, ncomp == 1 ? 1 : DG, out, s);
+            downloadSoA(io, tmpDG.p, ne, ncomp == 1 ? 1 : DG, out, s);
         } else if (n == "hice" || n == "cice" || (brittle && n == "damage")) {
             require(ncomp == 1 || ncomp == DG, "ncomp must be 1 or DG");
-            downloadSoA(scratch, n == "hice" ? h.p : (n == "cice" ? A.p : damage.p), ne, ncomp, out, s);
+            downloadSoA(io, n == "hice" ? h.p : (n == "cice" ? A.p : damage.p), ne, ncomp, out, s);
         } else if (n == "ssh") {
             require(ncomp == 1, "ssh is a DG0 field");
-            downloadSoA(scratch, ssh.p, ne, 1, out, s);
+            downloadSoA(io, ssh.p, ne, 1, out, s);
         } else if (const double* t = tensorRef(n)) {
             require(ncomp == 1 || ncomp == S, "ncomp must be 1 or S");
-            downloadSoA(scratch, t, ne, ncomp, out, s);
+            downloadSoA(io, t, ne, ncomp, out, s);
         } else {
             auto it = passive.find(n);
             require(it != passive.end(), "unknown field " + n);
@@ -3883,8 +3884,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
         need();
         double* c = cgRef(n);
         require(c != nullptr, "unknown CG vector " + n);
-        NSDG_HIP(hipMemcpyAsync(out, c, nn * sizeof(double), hipMemcpyDeviceToHost, s));
-        NSDG_HIP(hipStreamSynchronize(s));
+        io.toHost(out, c, nn * sizeof(double), s);
     }
     void setCG(const std::string& n, const double* in) override
     {
@@ -4829,7 +4829,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
         std::memcpy(buf.data(), &hd, sizeof hd);
         size_t off = sizeof(Header);
         for (auto& pr : stateParts()) {
-            NSDG_HIP(hipMemcpyAsync(buf.data() + off, pr.first, pr.second * sizeof(double), hipMemcpyDeviceToHost, s));
+            io.toHost(buf.data() + off, pr.first, pr.second * sizeof(double), s);
             off += pr.second * sizeof(double);
         }
         NSDG_HIP(hipStreamSynchronize(s));

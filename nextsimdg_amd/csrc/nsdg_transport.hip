@@ -13,7 +13,10 @@
 #include "nsdg_device.hpp"
 #include "nsdg_transport.hpp"
 
+#include <algorithm>
 #include <cstring>
+#include <exception>
+#include <thread>
 
 namespace nsdg {
 
@@ -709,31 +712,115 @@ __global__ void k_fill(double* p, size_t n, double v)
         p[t] = v;
 }
 
-void uploadSoA(DBuf<double>& scratch, const double* host, size_t n, int nc, double* dst, hipStream_t s)
+HostIO::~HostIO() { release(); }
+void HostIO::release()
+{
+    for (auto& e : done) {
+        if (e)
+            (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+    if (pinned)
+        (void)hipHostFree(pinned);
+    pinned = nullptr;
+    threads = 0;
+}
+void HostIO::reserve(int n)
+{
+    if (n <= threads)
+        return;
+    release();
+    NSDG_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), 2 * n * kSlot, hipHostMallocDefault));
+    for (int i = 0; i < 2 * n; ++i)
+        NSDG_HIP(hipEventCreateWithFlags(&done[i], hipEventDisableTiming));
+    threads = n;
+}
+// One thread's share of a copy, slot by slot through its two pinned slots.
+void HostIO::part(char* host, const char* dev, size_t bytes, int t, hipStream_t s)
+{
+    const size_t n = (bytes + kSlot - 1) / kSlot;
+    const auto size = [&](size_t i) { return std::min(kSlot, bytes - i * kSlot); };
+    const auto slot = [&](size_t i) { return pinned + (2 * t + (i & 1)) * kSlot; };
+    const auto issue = [&](size_t i) {
+        NSDG_HIP(hipMemcpyAsync(slot(i), dev + i * kSlot, size(i), hipMemcpyDeviceToHost, s));
+        NSDG_HIP(hipEventRecord(done[2 * t + (i & 1)], s));
+    };
+    for (size_t i = 0; i < std::min<size_t>(2, n); ++i)
+        issue(i);
+    for (size_t i = 0; i < n; ++i) {
+        NSDG_HIP(hipEventSynchronize(done[2 * t + (i & 1)]));
+        std::memcpy(host + i * kSlot, slot(i), size(i));
+        if (i + 2 < n)
+            issue(i + 2);
+    }
+}
+void HostIO::toHost(void* hostp, const void* src, size_t bytes, hipStream_t s)
+{
+    char* const host = static_cast<char*>(hostp);
+    const char* const dev = static_cast<const char*>(src);
+    if (bytes < kMinSplit) {
+        if (bytes)
+            NSDG_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
+        NSDG_HIP(hipStreamSynchronize(s));
+        return;
+    }
+    const int n = static_cast<int>(std::min<size_t>(kThreads, bytes / kSlot));
+    reserve(n);
+    const size_t share = ((bytes + n - 1) / n + 4095) & ~size_t(4095);
+    int device = 0;
+    NSDG_HIP(hipGetDevice(&device));
+    std::exception_ptr failed[kThreads];
+    const auto run = [&](int t) noexcept {
+        try {
+            const size_t lo = std::min(bytes, t * share), hi = std::min(bytes, lo + share);
+            NSDG_HIP(hipSetDevice(device));
+            if (hi > lo)
+                part(host + lo, dev + lo, hi - lo, t, s);
+        } catch (...) {
+            failed[t] = std::current_exception();
+        }
+    };
+    std::thread pool[kThreads];
+    for (int t = 1; t < n; ++t) {
+        try {
+            pool[t] = std::thread(run, t);
+        } catch (...) { // no more threads to be had: this one takes the share
+            run(t);
+        }
+    }
+    run(0);
+    for (int t = 1; t < n; ++t)
+        if (pool[t].joinable())
+            pool[t].join();
+    for (int t = 0; t < n; ++t)
+        if (failed[t]) {
+            (void)hipStreamSynchronize(s); // no copy may still be filling a slot
+            std::rethrow_exception(failed[t]);
+        }
+}
+void uploadSoA(HostIO& io, const double* host, size_t n, int nc, double* dst, hipStream_t s)
 {
     if (nc == 1) {
         NSDG_HIP(hipMemcpyAsync(dst, host, n * sizeof(double), hipMemcpyHostToDevice, s));
         return;
     }
-    if (scratch.n < n * nc)
-        scratch.alloc(n * nc);
-    scratch.upload(host, n * nc, s);
-    k_aos_to_soa<<<blocksFor(n * nc), kBlock, 0, s>>>(scratch.p, n, nc, dst);
+    if (io.scratch.n < n * nc)
+        io.scratch.alloc(n * nc);
+    io.scratch.upload(host, n * nc, s);
+    k_aos_to_soa<<<blocksFor(n * nc), kBlock, 0, s>>>(io.scratch.p, n, nc, dst);
     checkLaunch("aos_to_soa");
 }
-void downloadSoA(DBuf<double>& scratch, const double* src, size_t n, int nc, double* host, hipStream_t s)
+void downloadSoA(HostIO& io, const double* src, size_t n, int nc, double* host, hipStream_t s)
 {
     if (nc == 1) {
-        NSDG_HIP(hipMemcpyAsync(host, src, n * sizeof(double), hipMemcpyDeviceToHost, s));
-        NSDG_HIP(hipStreamSynchronize(s));
+        io.toHost(host, src, n * sizeof(double), s);
         return;
     }
-    if (scratch.n < n * nc)
-        scratch.alloc(n * nc);
-    k_soa_to_aos<<<blocksFor(n * nc), kBlock, 0, s>>>(src, n, nc, scratch.p);
+    if (io.scratch.n < n * nc)
+        io.scratch.alloc(n * nc);
+    k_soa_to_aos<<<blocksFor(n * nc), kBlock, 0, s>>>(src, n, nc, io.scratch.p);
     checkLaunch("soa_to_aos");
-    scratch.download(host, n * nc, s);
-    NSDG_HIP(hipStreamSynchronize(s));
+    io.toHost(host, io.scratch.p, n * nc * sizeof(double), s);
 }
 void deviceFill(double* p, size_t n, double v, hipStream_t s)
 {
@@ -823,7 +910,8 @@ template <int DG> struct TransportImpl final : TransportBase {
     Profiler& prof;
     int scheme = 2;
     int nXe, nYe;
-    DBuf<double> ops, vx, vy, nvX, nvY, tmpA, tmpB, raw, scratch;
+    DBuf<double> ops, vx, vy, nvX, nvY, tmpA, tmpB, raw, cgU, cgV;
+    HostIO io;
     CG2DGOps cg2dg[3];
 
     TransportImpl(DeviceMesh& m, hipStream_t st, Profiler& p)
@@ -857,8 +945,8 @@ template <int DG> struct TransportImpl final : TransportBase {
     double* vely() override { return vy.p; }
     void setVelocityHost(const double* hx, const double* hy) override
     {
-        uploadSoA(scratch, hx, mesh.ne, DG, vx.p, s);
-        uploadSoA(scratch, hy, mesh.ne, DG, vy.p, s);
+        uploadSoA(io, hx, mesh.ne, DG, vx.p, s);
+        uploadSoA(io, hy, mesh.ne, DG, vy.p, s);
         NSDG_HIP(hipStreamSynchronize(s));
     }
     void prepareAdvectionHost(int cg, const double* u, const double* v) override
@@ -867,12 +955,12 @@ template <int DG> struct TransportImpl final : TransportBase {
         if (cg2dg[cg].cg != cg)
             cg2dg[cg].build(cg, DG, mesh, s);
         const size_t ncg = static_cast<size_t>(cg * mesh.nx + 1) * (cg * mesh.ny + 1);
-        DBuf<double> du, dv;
-        du.alloc(ncg);
-        dv.alloc(ncg);
-        du.upload(u, ncg, s);
-        dv.upload(v, ncg, s);
-        cg2dg[cg].apply(mesh, du.p, vx.p, dv.p, vy.p, s, prof);
+        for (auto* b : { &cgU, &cgV }) // kept for the next velocity
+            if (b->n < ncg)
+                b->alloc(ncg);
+        cgU.upload(u, ncg, s);
+        cgV.upload(v, ncg, s);
+        cg2dg[cg].apply(mesh, cgU.p, vx.p, cgV.p, vy.p, s, prof);
         reinitNormalVelocity();
         NSDG_HIP(hipStreamSynchronize(s));
     }

@@ -203,14 +203,14 @@ class MEVPDynamicsKernel:
         check(self.lib.nsdg_dyn_set_field(self.h, name.encode(), dptr(a), int(ncomp)))
 
     def getDG0Data(self, name):
-        out = np.zeros(self.ne)
+        out = np.empty(self.ne)
         check(self.lib.nsdg_dyn_get_field(self.h, name.encode(), dptr(out), 1))
         return out
 
     def getDGData(self, name, ncomp=None):
         if ncomp is None:
             ncomp = self.S if name[0] in "se" and name[1:] in ("11", "12", "22") else self.dg
-        out = np.zeros(self.ne * ncomp)
+        out = np.empty(self.ne * ncomp)
         check(self.lib.nsdg_dyn_get_field(self.h, name.encode(), dptr(out), int(ncomp)))
         return out.reshape(self.ne, ncomp)
 
@@ -220,7 +220,7 @@ class MEVPDynamicsKernel:
 
     # ---- per-pass and support entries
     def get_cg(self, name):
-        out = np.zeros(self.ncg)
+        out = np.empty(self.ncg)
         check(self.lib.nsdg_dyn_get_cg(self.h, name.encode(), dptr(out)))
         return out
 
