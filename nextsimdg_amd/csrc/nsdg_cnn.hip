@@ -244,72 +244,117 @@ __global__ __launch_bounds__(kThreads) void k_loss(const float* z, const float* 
 
 // Weight gradient dW[co][ci][tap] = sum_p a(p + offset(tap))[ci] dz(p)[co] and bias
 // gradient sum_p dz(p)[co], as per-block partials part[block][tap][ci][co] (+ [co]).
-// A block takes 64-pixel row segments; wave w computes the (ci tile w / 2, co tile w % 2)
-// block of every tap.
-constexpr int SEG = 64;
+// A block takes bands of 4 rows by 64 pixels; wave w computes the (ci tile w / 2, co tile
+// w % 2) block of every tap, the waves of the first ci tile also the bias (a row of ones).
+// Its floor is one read of both images; it is bound by the latency of its loads against the
+// few matrix instructions of a band, so a band is as large as two blocks per CU allow (6
+// input rows for 4 gradient rows, held in registers while the previous band computes).
+// The band is staged channel-major, two pixels to a word. The three column shifts of a
+// row come from one 16-byte read and the word after it by funnel shifts: a fragment read
+// element by element at each shift was 144 two-byte LDS reads per 64 pixels and wave, and
+// the bias a serial loop of one wave. Rows of 36 words put the 16 channels of a fragment on
+// distinct banks. 16 images of 256 x 256: 106 -> 58 us with bands of one row, 37 us (3.6 TB/s)
+// with 4. Bands of one row on 768 blocks took 54 us; in an order that gives each XCD
+// neighbouring rows, on 512 blocks, 60 us.
+constexpr int SEG = 64, SEGW = SEG / 2 + 4, SROWS = 4; // pixels, words per channel row, rows
+__device__ __forceinline__ bf16x8 fragOf(uint32_t a, uint32_t b, uint32_t c, uint32_t d)
+{
+    return __builtin_bit_cast(bf16x8, make_uint4(a, b, c, d));
+}
 __global__ __launch_bounds__(kThreads) void k_wgrad(const uint16_t* __restrict__ a, const uint16_t* __restrict__ dz,
     int n, int ny, int nx, float* __restrict__ part)
 {
-    __shared__ uint16_t at[3][C][SEG + 2];
-    __shared__ __attribute__((aligned(16))) uint16_t gt[C][SEG];
+    __shared__ __attribute__((aligned(16))) uint32_t at[SROWS + 2][C][SEGW];
+    __shared__ __attribute__((aligned(16))) uint32_t gt[SROWS][C][SEGW];
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     const int mi = wave / 2, nj = wave % 2;
-    floatx4 acc[TAPS];
+    floatx4 acc[TAPS], accB { 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
     for (int t = 0; t < TAPS; ++t)
         acc[t] = floatx4 { 0.f, 0.f, 0.f, 0.f };
-    float db = 0.0f;
-    const int segs = (nx + SEG - 1) / SEG;
-    const long items = static_cast<long>(n) * ny * segs;
-    for (long it = blockIdx.x; it < items; it += gridDim.x) {
-        const int seg = static_cast<int>(it % segs);
-        const long rowId = it / segs;
-        const int y = static_cast<int>(rowId % ny);
-        const long img = rowId / ny;
-        const int x0 = SEG * seg;
-        __syncthreads();
-        for (int q = threadIdx.x; q < 3 * (SEG + 2) * 4; q += kThreads) {
-            const int cg = q % 4, px = (q / 4) % (SEG + 2), row = q / (4 * (SEG + 2));
-            const int xp = x0 - 1 + px, yp = y - 1 + row;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (xp >= 0 && xp < nx && yp >= 0 && yp < ny)
-                v = *reinterpret_cast<const uint4*>(a + ((img * ny + yp) * nx + xp) * C + 8 * cg);
-            const uint32_t wv[4] = { v.x, v.y, v.z, v.w };
+    const int segs = (nx + SEG - 1) / SEG, bands = (ny + SROWS - 1) / SROWS;
+    const long items = static_cast<long>(n) * bands * segs;
+    // loading tasks: 8 channels of a pixel pair, of the input's rows (with the halo pixel on
+    // either side) and then of the gradient's
+    constexpr int PAIRS = SEG / 2 + 1, ATASKS = (SROWS + 2) * PAIRS * 4, TASKS = ATASKS + SROWS * (SEG / 2) * 4;
+    constexpr int PER = (TASKS + kThreads - 1) / kThreads;
+    uint4 v[PER][2];
+    const auto load = [&](long it) {
+        const int x0 = SEG * static_cast<int>(it % segs);
+        const long bandId = it / segs, img = bandId / bands;
+        const int y0 = SROWS * static_cast<int>(bandId % bands);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                at[row][8 * cg + 2 * k][px] = static_cast<uint16_t>(wv[k] & 0xFFFFu);
-                at[row][8 * cg + 2 * k + 1][px] = static_cast<uint16_t>(wv[k] >> 16);
+        for (int k = 0; k < PER; ++k) {
+            const int q = threadIdx.x + k * kThreads, cg = q % 4;
+            const bool isA = q < ATASKS;
+            const int r = (isA ? q : q - ATASKS) / 4, row = r / (isA ? PAIRS : SEG / 2), pair = r % (isA ? PAIRS : SEG / 2);
+            const int xp = isA ? x0 - 1 + 2 * pair : x0 + 2 * pair, yp = y0 + row - (isA ? 1 : 0);
+            const uint16_t* const src = (isA ? a : dz) + ((img * ny + yp) * nx + xp) * C + 8 * cg;
+            const bool in = q < TASKS && yp >= 0 && yp < ny;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                v[k][h] = make_uint4(0, 0, 0, 0);
+                if (in && xp + h >= 0 && xp + h < nx)
+                    v[k][h] = *reinterpret_cast<const uint4*>(src + h * C);
             }
         }
-        for (int q = threadIdx.x; q < SEG * 4; q += kThreads) {
-            const int cg = q % 4, px = q / 4;
-            const int xp = x0 + px;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (xp < nx)
-                v = *reinterpret_cast<const uint4*>(dz + (rowId * nx + xp) * C + 8 * cg);
-            const uint32_t wv[4] = { v.x, v.y, v.z, v.w };
+    };
+    const auto stage = [&] {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                gt[8 * cg + 2 * k][px] = static_cast<uint16_t>(wv[k] & 0xFFFFu);
-                gt[8 * cg + 2 * k + 1][px] = static_cast<uint16_t>(wv[k] >> 16);
+        for (int k = 0; k < PER; ++k) {
+            const int q = threadIdx.x + k * kThreads, cg = q % 4;
+            if (q >= TASKS)
+                continue;
+            const bool isA = q < ATASKS;
+            const int r = (isA ? q : q - ATASKS) / 4, row = r / (isA ? PAIRS : SEG / 2), pair = r % (isA ? PAIRS : SEG / 2);
+            uint32_t* const dst = isA ? &at[row][8 * cg][pair] : &gt[row][8 * cg][pair];
+            const uint32_t lo[4] = { v[k][0].x, v[k][0].y, v[k][0].z, v[k][0].w };
+            const uint32_t hi[4] = { v[k][1].x, v[k][1].y, v[k][1].z, v[k][1].w };
+#pragma unroll
+            for (int c = 0; c < 4; ++c) { // channels 2 c, 2 c + 1 of the pair, left pixel in the low half
+                dst[(2 * c) * SEGW] = (lo[c] & 0xFFFFu) | (hi[c] << 16);
+                dst[(2 * c + 1) * SEGW] = (lo[c] >> 16) | (hi[c] & 0xFFFF0000u);
             }
         }
+    };
+    constexpr uint32_t one2 = 0x3F803F80u; // two bfloat16 ones
+    long it = blockIdx.x;
+    if (it < items)
+        load(it);
+    for (; it < items; it += gridDim.x) {
+        __syncthreads(); // the previous segment is consumed
+        stage();
+        if (it + gridDim.x < items)
+            load(it + gridDim.x);
         __syncthreads();
-        if (threadIdx.x < C)
-            for (int px = 0; px < SEG; ++px)
-                db += fromBF16(gt[threadIdx.x][px]);
 #pragma unroll
         for (int kc = 0; kc < SEG / 32; ++kc) {
-            const bf16x8 b = frag(&gt[16 * nj + lane % 16][32 * kc + 8 * (lane / 16)]);
+            const int w0 = 16 * kc + 4 * (lane / 16);
+            bf16x8 b[SROWS];
 #pragma unroll
-            for (int t = 0; t < TAPS; ++t) {
-                const int dyi = t / 3, dxi = t % 3;
-                const uint16_t* src = &at[dyi][16 * mi + lane % 16][32 * kc + 8 * (lane / 16) + dxi];
-                bf16x8 av;
+            for (int y = 0; y < SROWS; ++y) {
+                const uint4 g = *reinterpret_cast<const uint4*>(&gt[y][16 * nj + lane % 16][w0]);
+                b[y] = fragOf(g.x, g.y, g.z, g.w);
+                if (mi == 0)
+                    accB = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fragOf(one2, one2, one2, one2), b[y], accB, 0, 0, 0);
+            }
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    av[i] = __builtin_bit_cast(__bf16, src[i]);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b, acc[t], 0, 0, 0);
+            for (int r = 0; r < SROWS + 2; ++r) { // input row y0 - 1 + r: row r - y of the stencil about y0 + y
+                const uint32_t* const src = &at[r][16 * mi + lane % 16][w0];
+                const uint4 w = *reinterpret_cast<const uint4*>(src);
+                const uint32_t w4 = src[4];
+                const bf16x8 left = fragOf(w.x, w.y, w.z, w.w), right = fragOf(w.y, w.z, w.w, w4);
+                const bf16x8 mid = fragOf(__builtin_amdgcn_alignbit(w.y, w.x, 16), __builtin_amdgcn_alignbit(w.z, w.y, 16),
+                    __builtin_amdgcn_alignbit(w.w, w.z, 16), __builtin_amdgcn_alignbit(w4, w.w, 16));
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const int y = r - k;
+                    if (y < 0 || y >= SROWS)
+                        continue;
+                    acc[3 * k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(left, b[y], acc[3 * k], 0, 0, 0);
+                    acc[3 * k + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mid, b[y], acc[3 * k + 1], 0, 0, 0);
+                    acc[3 * k + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(right, b[y], acc[3 * k + 2], 0, 0, 0);
+                }
             }
         }
     }
@@ -321,29 +366,43 @@ __global__ __launch_bounds__(kThreads) void k_wgrad(const uint16_t* __restrict__
             const int ci = 16 * mi + 4 * (lane / 16) + i, co = 16 * nj + lane % 16;
             P[(t * C + ci) * C + co] = acc[t][i];
         }
-    if (threadIdx.x < C)
-        P[WSZ + threadIdx.x] = db;
+    if (mi == 0 && lane < 16) // every row of the product with ones is the sum
+        P[WSZ + 16 * nj + lane] = accB[0];
 }
-// Sum of the partials in block order, into the parameter layout [co][ci][tap], bias. The
-// loads go out 16 at a time ahead of their (in-order) additions.
-__global__ void k_wgrad_reduce(const float* part, int nb, float* g)
+// Sum of the partials, into the parameter layout [co][ci][tap], bias. A block takes
+// kSumElems parameters, its threads in kSlices slices of the partials: each adds its slice in
+// block order, 8 loads ahead, and the slices are added in order (the same sum in every
+// run). One thread per parameter over all 512 partials left most of the chip idle: 22 -> 5.6 us.
+constexpr int kSumElems = 32, kSlices = kThreads / kSumElems;
+__global__ __launch_bounds__(kThreads) void k_wgrad_reduce(const float* part, int nb, float* g)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= PSZ)
-        return;
+    __shared__ float sh[kSlices][kSumElems];
+    const int k = threadIdx.x % kSumElems, slice = threadIdx.x / kSumElems;
+    const int e = blockIdx.x * kSumElems + k;
+    const int per = (nb + kSlices - 1) / kSlices, b1 = min(nb, (slice + 1) * per);
     float sum = 0.0f;
-    int b = 0;
-    for (; b + 16 <= nb; b += 16) {
-        float v[16];
+    if (e < PSZ) {
+        int b = slice * per;
+        for (; b + 8 <= b1; b += 8) {
+            float v[8];
 #pragma unroll
-        for (int k = 0; k < 16; ++k)
-            v[k] = part[static_cast<size_t>(b + k) * PSZ + e];
+            for (int i = 0; i < 8; ++i)
+                v[i] = part[static_cast<size_t>(b + i) * PSZ + e];
 #pragma unroll
-        for (int k = 0; k < 16; ++k)
-            sum += v[k];
+            for (int i = 0; i < 8; ++i)
+                sum += v[i];
+        }
+        for (; b < b1; ++b)
+            sum += part[static_cast<size_t>(b) * PSZ + e];
     }
-    for (; b < nb; ++b)
-        sum += part[static_cast<size_t>(b) * PSZ + e];
+    sh[slice][k] = sum;
+    __syncthreads();
+    if (slice != 0 || e >= PSZ)
+        return;
+    sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kSlices; ++i)
+        sum += sh[i][k];
     if (e < WSZ) {
         const int t = e / (C * C), ci = (e / C) % C, co = e % C;
         g[(co * C + ci) * TAPS + t] = sum;
@@ -488,13 +547,14 @@ double Net::lossGrad(const uint16_t* x, const float* t, const float* w, int n, i
         k_loss<<<nbLoss, kThreads, 0, s>>>(out.p, t, w, npix, dz0.p, lossPart.p);
         checkLaunch("cnn_loss");
     }
-    const long items = static_cast<long>(n) * ny * ((nx + SEG - 1) / SEG);
+    const long items = static_cast<long>(n) * ((ny + SROWS - 1) / SROWS) * ((nx + SEG - 1) / SEG);
     const unsigned nbW = gridFor(items, 1, kWgradBlocks);
     auto wgrad = [&](const uint16_t* a, const uint16_t* dz, int layer) {
         Timed tm(prof, s, "cnn_wgrad");
         k_wgrad<<<nbW, kThreads, 0, s>>>(a, dz, n, ny, nx, part.p);
         checkLaunch("cnn_wgrad");
-        k_wgrad_reduce<<<(PSZ + 255) / 256, 256, 0, s>>>(part.p, static_cast<int>(nbW), grad.p + layer * PSZ);
+        k_wgrad_reduce<<<(PSZ + kSumElems - 1) / kSumElems, kThreads, 0, s>>>(
+            part.p, static_cast<int>(nbW), grad.p + layer * PSZ);
         checkLaunch("cnn_wgrad_reduce");
     };
     // layer 3 (linear output): dz0 = dL/dz4

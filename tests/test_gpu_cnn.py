@@ -69,6 +69,22 @@ def test_loss_and_gradients_match_oracle():
     assert np.all(gl[cnn.OUT:] == 0.0)
 
 
+# Edges of the weight gradient's 4-row by 64-pixel bands, one band to more bands than blocks.
+# The tolerance above: one flipped BF16 rounding is 2^-8 of its term, so 3.9e-3 even where a
+# single term makes the sum; a lost band, row or halo pixel is at least 1/sqrt(516) = 4e-2.
+@pytest.mark.parametrize("n,ny,nx", [(1, 1, 16), (1, 3, 48), (3, 4, 64), (2, 5, 80), (1, 9, 144), (2, 1030, 16)])
+def test_gradients_at_band_edges_match_oracle(n, ny, nx):
+    net, p, x, xh, t, w = _setup(4, n, ny, nx)
+    w[:] = 1.0
+    _, g = net.loss_grad(x, _dev(t), _dev(w), want_grad=True)
+    _, rg = cnn.loss_grad(p, xh, t, w, emulate=True)
+    for l in range(cnn.LAYERS):
+        sl = slice(l * cnn.PSZ, (l + 1) * cnn.PSZ)
+        e = _rel(g[sl], rg[sl])
+        _say(f"  {n}x{ny}x{nx} layer {l} gradient rel L2 {e:.2e}")
+        assert e < 5e-3, (l, e)
+
+
 def test_adam_step_matches_oracle():
     net, p, x, _, t, w = _setup(3)
     _, g = net.loss_grad(x, _dev(t), _dev(w), want_grad=True)
