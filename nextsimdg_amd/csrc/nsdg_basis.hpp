@@ -125,28 +125,6 @@ template <int D, int G> constexpr Mat<D, G * G> make_psil()
             m.a[i][q] = dg_basis(i, lagrange_point(G, q % G), lagrange_point(G, q / G));
     return m;
 }
-// PSIe<E,G>
-template <int E, int G> constexpr Mat<E, G> make_psie()
-{
-    Mat<E, G> m {};
-    for (int i = 0; i < E; ++i)
-        for (int q = 0; q < G; ++q)
-            m.a[i][q] = edge_basis(i, gauss_point(G, q));
-    return m;
-}
-// PSIe_w<D,G,side>: [q][i], side 0 bottom, 1 right, 2 top, 3 left
-template <int D, int G, int SIDE> constexpr Mat<G, D> make_psiew()
-{
-    Mat<G, D> m {};
-    for (int q = 0; q < G; ++q)
-        for (int i = 0; i < D; ++i) {
-            const double t = gauss_point(G, q);
-            const double x = SIDE == 0 ? t : (SIDE == 1 ? 1.0 : (SIDE == 2 ? t : 0.0));
-            const double y = SIDE == 0 ? 0.0 : (SIDE == 1 ? t : (SIDE == 2 ? 1.0 : t));
-            m.a[q][i] = gauss_weight(G, q) * dg_basis(i, x, y);
-        }
-    return m;
-}
 // PHI<CG,G>, PHIx<CG,G>, PHIy<CG,G>
 template <int CG, int G, int WHICH> constexpr Mat<cgdofs(CG), G * G> make_phi()
 {
@@ -173,37 +151,6 @@ template <int D, int G> struct Psi {
 template <int D, int G> struct PsiL {
     static constexpr Mat<D, G * G> v = make_psil<D, G>();
 };
-template <int E, int G> struct PsiE {
-    static constexpr Mat<E, G> v = make_psie<E, G>();
-};
-template <int D, int G> struct PsiEW {
-    static constexpr Mat<G, D> b = make_psiew<D, G, 0>();
-    static constexpr Mat<G, D> r = make_psiew<D, G, 1>();
-    static constexpr Mat<G, D> t = make_psiew<D, G, 2>();
-    static constexpr Mat<G, D> l = make_psiew<D, G, 3>();
-};
-// Projection onto the DG stress basis on an affine element: M^-1 (PSI diag(w J)) with the
-// element mass M = J diag(m), m_s = sum_q w_q PSI_s(q)^2 (the basis is orthogonal under the
-// Gauss rule), so iMJwPSI[s][q] = PSI_s(q) w_q / m_s, independent of the element.
-template <int S, int G> constexpr Mat<S, G * G> make_bproj()
-{
-    Mat<S, G * G> m {};
-    for (int s = 0; s < S; ++s) {
-        double ms = 0;
-        for (int q = 0; q < G * G; ++q) {
-            const double p = dg_basis(s, gauss_point(G, q % G), gauss_point(G, q / G));
-            ms += gauss_weight(G, q % G) * gauss_weight(G, q / G) * p * p;
-        }
-        for (int q = 0; q < G * G; ++q)
-            m.a[s][q] = dg_basis(s, gauss_point(G, q % G), gauss_point(G, q / G))
-                * (gauss_weight(G, q % G) * gauss_weight(G, q / G)) / ms;
-    }
-    return m;
-}
-template <int S, int G> struct BProj {
-    static constexpr Mat<S, G * G> v = make_bproj<S, G>();
-};
-
 template <int CG, int G> struct Phi {
     static constexpr Mat<cgdofs(CG), G * G> v = make_phi<CG, G, 0>();
     static constexpr Mat<cgdofs(CG), G * G> x = make_phi<CG, G, 1>();

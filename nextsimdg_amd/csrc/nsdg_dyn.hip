@@ -1,18 +1,19 @@
 // mEVP momentum/rheology subcycle and the per-timestep driver on gfx950.
 //
-// One mEVP subcycle is two bulk-synchronous HBM passes:
-//  * element pass: strain rate from the 9 (CG2) / 4 (CG1) velocity nodes, the mEVP
+// One mEVP subcycle is two steps, a block of one launch taking a tile through both (on
+// meshes with periodic segments they are separate launches):
+//  * element update: strain rate from the 9 (CG2) / 4 (CG1) velocity nodes, the mEVP
 //    stress relaxation at the Gauss points and its projection back to the DG stress
 //    basis, in registers; reads u, v, h, A, sigma, writes sigma. Strain never
 //    touches HBM.
-//  * node pass: a 256-thread block takes a tile of elements plus a one-element halo,
+//  * node update: the block takes a tile of elements plus a one-element halo,
 //    computes each element's weak-divergence contributions to its CG nodes into LDS,
 //    then every CG node of the tile sums its <= 4 contributions in the reference's
 //    two-colour stripe order (atomic-free, deterministic) and applies the FP64
 //    implicit velocity update and the Dirichlet zero.
-// On a uniform mesh one copy of each element operator is read with wave-uniform
-// addresses (scalar loads through the constant cache); otherwise operators are
-// streamed per element, k-major. Per-step set-up (CG2DG, normal velocities, the two
+// On a uniform mesh the operators are literals and five scalars of the element map; on
+// other meshes they are formed from per-element geometry (streamed as k-major tables by
+// the separate launches only). Per-step set-up (CG2DG, normal velocities, the two
 // transported fields, limiters, DG2CG, sea-surface-height gradient) are further
 // element- or node-parallel kernels. Nothing runs on the host between launches.
 //
@@ -1448,9 +1449,7 @@ __device__ __forceinline__ void divergenceLocal(const NodeArgs& a, int e, double
 // tx = Dxi p1 + Deta q1 and ty = Dxi p2 + Deta q2, with p1 = |J| (xi_x s11 + xi_y s12),
 // q1 = |J| (eta_x s11 + eta_y s12), p2 = |J| (xi_x s12 + xi_y s22), q2 = |J| (eta_x s12 +
 // eta_y s22): the reference's Gauss-point form (divS1, divS2: ParametricMap.cpp:269-271) with the
-// quadrature carried out in the literals. The matrices are the Gauss rule's values (exact
-// for these polynomial degrees), folded to constants; entries that vanish analytically
-// are exact zeros and are skipped (40 of 72 nonzero per matrix for CG2).
+// quadrature (exact for these polynomial degrees) carried out in the literals.
 // t = Dxi p + Deta q with p = xi_x a + xi_y b, q = eta_x a + eta_y b (|J| in the scalars).
 // Both matrices are products of 1-D integrals of a CG function (or its derivative) against
 // a Legendre polynomial, contracted one direction after the other: with the CG2 functions
@@ -1938,10 +1937,11 @@ template <int CG, int DG> __global__ __launch_bounds__(kBlock) void k_residual_f
 // the node velocities (coalesced, into an LDS window that the element and node updates
 // share), the strength and the nodes' frozen terms at the start, the previous stress between
 // the strain and the rheology. Strength and frozen terms stay in registers for sub-step 2
-// (252 VGPRs, 68 KB of LDS: two blocks per CU) instead of being read again by three blocks
+// (214 VGPRs, 68 KB of LDS: two blocks per CU) instead of being read again by three blocks
 // of 160 VGPRs, each phase waiting for its own loads. Per launch: 24 x 24 box 15.8 -> 14.6
 // us, CG1 128 x 128 8.1 -> 7.2, 2048 x 2048 1106 -> 975, 512 x 512 70.6 -> 70.0 (its 1600
-// tiles are 3.1 rounds of 512 blocks). The same registers filled in another order, frozen
+// tiles are 3.1 rounds of 512 blocks); with the sum factorisations in even and odd parts
+// 13.0, 7.0, 899 and 62.8. The same registers filled in another order, frozen
 // terms first, took 96 us at 512 x 512.
 template <int CG, class R> struct PairTile {
     static constexpr int TX = sizeof(R) == 8 ? 13 : 29, TY = 13;
