@@ -495,6 +495,7 @@ void Net::reserve(size_t npix)
 {
     if (npix <= pixels)
         return;
+    pixels = 0; // until all of them are there
     for (int l = 1; l < LAYERS; ++l)
         act[l].alloc(npix * C);
     dz0.alloc(npix * C);

@@ -4606,7 +4606,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
     void saveStart() override
     {
         need();
-        if (uStart.n != nn) {
+        if (sigStart.n != sig.n) { // the last of the three to be allocated
             uStart.alloc(nn);
             vStart.alloc(nn);
             sigStart.alloc(sig.n);
@@ -4645,7 +4645,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
     }
     void allocPrecision()
     {
-        if (precision == NSDG_PREC_FP32 && ready && sigF.n != 3 * S * ne) {
+        if (precision == NSDG_PREC_FP32 && ready && strengthF.n != static_cast<size_t>(L::Q) * ne) {
             sigF.alloc(3 * S * ne);
             sigFAlt.alloc(3 * S * ne);
             strengthF.alloc(static_cast<size_t>(L::Q) * ne);

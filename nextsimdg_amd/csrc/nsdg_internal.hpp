@@ -59,9 +59,9 @@ template <class T> struct DBuf {
     void alloc(size_t count)
     {
         release();
-        n = count;
-        if (n)
-            NSDG_HIP(hipMalloc(reinterpret_cast<void**>(&p), n * sizeof(T)));
+        if (count)
+            NSDG_HIP(hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T)));
+        n = count; // only with the memory: a buffer that is kept is tested by its size
     }
     void upload(const T* h, size_t count, hipStream_t s, size_t offset = 0)
     {

@@ -853,24 +853,24 @@ void deviceCopy(double* dst, const double* src, size_t n, hipStream_t s)
 
 void CG2DGOps::build(int cg_, int dg_, const DeviceMesh& mesh, hipStream_t s)
 {
-    cg = cg_;
-    dg = dg_;
     const int nOps = mesh.uniform ? 1 : static_cast<int>(mesh.ne);
-    const int N = cgdofs(cg);
-    ops.alloc(static_cast<size_t>(dg) * N * nOps);
+    cg = 0; // until the operators are there
+    ops.alloc(static_cast<size_t>(dg_) * cgdofs(cg_) * nOps);
     const MeshView mv = view(mesh);
     auto go = [&](auto kern) {
         kern<<<blocksFor(nOps), kBlock, 0, s>>>(mv, nOps, ops.p);
         checkLaunch("cg2dg_ops");
     };
-    if (cg == 1 && dg == 1) go(k_cg2dg_ops<1, 1>);
-    else if (cg == 1 && dg == 3) go(k_cg2dg_ops<1, 3>);
-    else if (cg == 1 && dg == 6) go(k_cg2dg_ops<1, 6>);
-    else if (cg == 2 && dg == 1) go(k_cg2dg_ops<2, 1>);
-    else if (cg == 2 && dg == 3) go(k_cg2dg_ops<2, 3>);
-    else if (cg == 2 && dg == 6) go(k_cg2dg_ops<2, 6>);
-    else if (cg == 2 && dg == 8) go(k_cg2dg_ops<2, 8>);
+    if (cg_ == 1 && dg_ == 1) go(k_cg2dg_ops<1, 1>);
+    else if (cg_ == 1 && dg_ == 3) go(k_cg2dg_ops<1, 3>);
+    else if (cg_ == 1 && dg_ == 6) go(k_cg2dg_ops<1, 6>);
+    else if (cg_ == 2 && dg_ == 1) go(k_cg2dg_ops<2, 1>);
+    else if (cg_ == 2 && dg_ == 3) go(k_cg2dg_ops<2, 3>);
+    else if (cg_ == 2 && dg_ == 6) go(k_cg2dg_ops<2, 6>);
+    else if (cg_ == 2 && dg_ == 8) go(k_cg2dg_ops<2, 8>);
     else throw Error(NSDG_ERR_UNSUPPORTED, "unsupported (cg, dg) for CG2DG");
+    cg = cg_;
+    dg = dg_;
 }
 
 void CG2DGOps::apply(const DeviceMesh& mesh, const double* src, double* dst, const double* src2, double* dst2,
