@@ -435,11 +435,13 @@ __device__ __forceinline__ uint32_t after(uint32_t off, double x)
     return off;
 }
 template <class T> __device__ __forceinline__ T ldAt(const T* base, uint32_t off) { return fieldAt(base, off); }
-// A double2 as its two halves (adjacent: the compiler can issue one 16-byte load).
-__device__ __forceinline__ double2 ld2At(const double2* base, uint32_t off)
+// Entry n of a double2 field as its two halves (adjacent: the compiler can issue one 16-byte
+// load). The address in 64 bits: the byte offset of a CG node passes 2^32 at n = 2^28.
+__device__ __forceinline__ double2 ld2At(const double2* base, uint32_t n)
 {
-    const double* b = reinterpret_cast<const double*>(base);
-    return make_double2(ldAt(b, off), ldAt(b, off + 8u));
+    const auto b = reinterpret_cast<const __attribute__((address_space(1))) double*>(
+        reinterpret_cast<uint64_t>(base) + (static_cast<uint64_t>(n) << 4));
+    return make_double2(b[0], b[1]);
 }
 constexpr int kXCD = 8;
 __device__ __forceinline__ int xcdTile(int b, int ntiles)

@@ -1565,14 +1565,14 @@ __device__ __forceinline__ void loadFrozen(const NodeArgs& a, int n, NodeFz& in)
     in.cf = a.cf[n];
     in.qf = a.qf[n];
 }
-// The same with scalar field bases and 32-bit byte offsets (node n < 2^29).
+// The same with scalar field bases and 32-bit byte offsets for u and v (node n < 2^29).
 __device__ __forceinline__ void loadFrozenAt(const NodeArgs& a, uint32_t n, NodeFz& in)
 {
     in.u = ldAt(a.u, n * 8u);
     in.v = ldAt(a.v, n * 8u);
-    in.ocn = ld2At(a.ocn, n * 16u);
-    in.cf = ld2At(a.cf, n * 16u);
-    in.qf = ld2At(a.qf, n * 16u);
+    in.ocn = ld2At(a.ocn, n);
+    in.cf = ld2At(a.cf, n);
+    in.qf = ld2At(a.qf, n);
 }
 __device__ __forceinline__ void momentumFrozen(const NodeArgs& a, const NodeFz& in, double dSx, double dSy, double& un,
     double& vn)
@@ -1970,9 +1970,9 @@ struct MevpNodeWindow {
         const int l = (nix - x0) + nw * (niy - y0);
         in.u = uS[l];
         in.v = vS[l];
-        in.ocn = ld2At(a.ocn, static_cast<uint32_t>(n) * 16u);
-        in.cf = ld2At(a.cf, static_cast<uint32_t>(n) * 16u);
-        in.qf = ld2At(a.qf, static_cast<uint32_t>(n) * 16u);
+        in.ocn = ld2At(a.ocn, static_cast<uint32_t>(n));
+        in.cf = ld2At(a.cf, static_cast<uint32_t>(n));
+        in.qf = ld2At(a.qf, static_cast<uint32_t>(n));
     }
     __device__ __forceinline__ void update(const NodeArgs& a, const In& in, int, bool, double dx, double dy,
         double& un, double& vn) const
@@ -2048,9 +2048,9 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : 1))) void k_mevp_pair(Fu
             fzLive[b] = i < NWH && nix >= 0 && nix <= CG * a.nx && niy >= 0 && niy <= CG * a.ny;
             const uint32_t n = fzLive[b] ? static_cast<uint32_t>(nix + row * niy) : 0u;
             fzDir[b] = ldAt(a.dirNode, n) != 0;
-            fzOcn[b] = ld2At(a.ocn, n * 16u);
-            fzCf[b] = ld2At(a.cf, n * 16u);
-            fzQf[b] = ld2At(a.qf, n * 16u);
+            fzOcn[b] = ld2At(a.ocn, n);
+            fzCf[b] = ld2At(a.cf, n);
+            fzQf[b] = ld2At(a.qf, n);
         }
 #pragma unroll
         for (int b = 0; b < NB0; ++b) {
@@ -3605,7 +3605,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
         nn1 = static_cast<size_t>(mesh.nx + 1) * (mesh.ny + 1);
         // the kernels index CG nodes with 32-bit ints (the mesh checks elements and vertices)
         require(nn < (size_t(1) << 31), "too many CG nodes for 32-bit node indices", NSDG_ERR_ARG);
-        // the one-pass kernels address element fields and CG nodes with 32-bit byte offsets
+        // the one-pass kernels address 8-byte element and node fields with 32-bit byte offsets
         // from scalar field bases (2^29 CG2 nodes: a 11585^2 mesh, ~210 GB of FP64 state)
         require(ne < (size_t(1) << 29), "meshes need fewer than 2^29 elements", NSDG_ERR_ARG);
         require(nn < (size_t(1) << 29), "meshes need fewer than 2^29 CG nodes", NSDG_ERR_ARG);
