@@ -141,9 +141,10 @@ template <int CG> __global__ void k_momentum_ops(MeshView m, int nOps, double* o
 // Reciprocal, reciprocal square root, square root and quotient of the subcycle kernels: the
 // hardware's estimates (about 24 bits) refined by Newton steps to an ulp, without the range
 // scaling and special-case selects of the general functions (half their instructions; the
-// element and node updates run 9 and 4 to 8 of them per element). Arguments are normal
-// numbers away from the ends of the range: Jacobians and their weights, Delta^2 >= DeltaMin^2,
-// squared speeds, the momentum denominators.
+// element and node updates run 9 and 4 to 8 of them per element). Arguments of the
+// reciprocals are normal numbers away from the ends of the range (Jacobians and their weights,
+// Delta^2 >= DeltaMin^2, the momentum denominators) or NaN, which passes through; zero and
+// infinity give NaN.
 __device__ __forceinline__ double reciprocal(double x)
 {
     double r = __builtin_amdgcn_rcp(x);
@@ -169,11 +170,12 @@ __device__ __forceinline__ double rsq(double x)
     return fma(y * e, fma(0.375, e, 0.5), y);
 }
 __device__ __forceinline__ float rsq(float x) { return rsqrtf(x); }
-// sqrt(x) for x >= 0; below 1e-280 (speeds of 1e-140 m/s) it returns 1e-140.
+// sqrt(x) for x >= 0, with an absolute error of 1e-140 below 1e-280. NaN passes through (the
+// lower bound enters the estimate only): a velocity component that is not a number reaches
+// the other one through the drag. Infinity gives NaN.
 __device__ __forceinline__ double squareRoot(double x)
 {
-    x = fmax(x, 1e-280);
-    const double y = __builtin_amdgcn_rsq(x);
+    const double y = __builtin_amdgcn_rsq(fmax(x, 1e-280));
     double g = x * y, h = 0.5 * y;
     const double r = fma(-h, g, 0.5);
     g = fma(g, r, g);
