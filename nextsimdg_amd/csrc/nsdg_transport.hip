@@ -758,7 +758,12 @@ void HostIO::toHost(void* hostp, const void* src, size_t bytes, hipStream_t s)
 {
     char* const host = static_cast<char*>(hostp);
     const char* const dev = static_cast<const char*>(src);
-    if (bytes < kMinSplit) {
+    // page-locked or device memory of the caller's: the copy engine writes it itself
+    hipPointerAttribute_t at {};
+    const bool known = bytes >= kMinSplit && hipPointerGetAttributes(&at, hostp) == hipSuccess
+        && at.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError(); // asking about ordinary memory is no error
+    if (bytes < kMinSplit || known) {
         if (bytes)
             NSDG_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
         NSDG_HIP(hipStreamSynchronize(s));
