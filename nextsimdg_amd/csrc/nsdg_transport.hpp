@@ -35,15 +35,20 @@ struct TransportBase {
 // Copies from the device to host memory, done when the call returns, and the device scratch
 // of the layout conversion. Of one handle, so used by one thread at a time.
 // The runtime copies into pageable memory through its own staging, one chunk and one core
-// at a time: 7 GB/s into fresh pages. From kMinSplit bytes up the range is split over a few
-// threads, each with two pinned slots, one filled by the copy engine while a core empties
-// the other; smaller copies stay with the runtime (starting the threads would cost what
-// they save). The four cell means of a 2048 x 2048 step: 18 -> 10 ms, of a 512 x 512 step
-// 0.08 ms less. Uploads stay with the runtime: it reads pageable memory faster (preparing
-// the 512 x 512 box took 15 ms through the slots, 11 without).
+// at a time. From kMinSplit bytes up the range is split over a few threads, each with two
+// pinned slots, one filled by the copy engine while a core empties the other. Plain against
+// split, into fresh pages (whose faults the threads share): 8 MiB 2.2 -> 1.2 to 1.5 ms, 32 MiB
+// 8.9 -> 5.4; into pages in use: 4 MiB 0.23 -> 0.24, 8 MiB 0.47 -> 0.44, 32 MiB 1.8 -> 1.6; the
+// first copy of a handle, which pins its slots, into pages in use: 4 MiB 0.27 -> 0.32, 8 MiB
+// 0.53 -> 0.54, 16 MiB 1.02 -> 0.93. Below 8 MiB a copy stays with the runtime; a thread
+// takes at least 4 MiB, so that a copy pays for its slots; eight threads copied no faster
+// than four and took twice as long to pin theirs. Slots of 256 KiB: 32 MiB 2.4 ms.
+// Page-locked and device destinations stay with the runtime (2048 x 2048 cell means 0.6 ms),
+// and so do uploads: it reads pageable memory faster (preparing the 512 x 512 box took 15
+// ms through the slots, 11 without).
 struct HostIO {
-    static constexpr size_t kMinSplit = size_t(1) << 20, kSlot = size_t(1) << 19;
-    static constexpr int kThreads = 8;
+    static constexpr size_t kMinSplit = size_t(1) << 23, kSlot = size_t(1) << 19, kMinShare = 8 * kSlot;
+    static constexpr int kThreads = 4;
     DBuf<double> scratch;
     HostIO() = default;
     HostIO(const HostIO&) = delete;
