@@ -69,10 +69,11 @@ def test_loss_and_gradients_match_oracle():
     assert np.all(gl[cnn.OUT:] == 0.0)
 
 
-# Edges of the weight gradient's 4-row by 64-pixel bands, one band to more bands than blocks.
-# The tolerance above: one flipped BF16 rounding is 2^-8 of its term, so 3.9e-3 even where a
-# single term makes the sum; a lost band, row or halo pixel is at least 1/sqrt(516) = 4e-2.
-@pytest.mark.parametrize("n,ny,nx", [(1, 1, 16), (1, 3, 48), (3, 4, 64), (2, 5, 80), (1, 9, 144), (2, 1030, 16)])
+# Edges of the weight gradient's 4-row by 64-pixel bands. The tolerance above: one flipped BF16
+# rounding is 2^-8 of its term, so 3.9e-3 even where a single term makes the sum. Of the 9 taps
+# of at most 1296 pixels, a lost halo pixel of a tap is 1/sqrt(9 * 1296) = 9e-3 or more, a row
+# or a band more than that.
+@pytest.mark.parametrize("n,ny,nx", [(1, 1, 16), (1, 3, 48), (3, 4, 64), (2, 5, 80), (1, 9, 144)])
 def test_gradients_at_band_edges_match_oracle(n, ny, nx):
     net, p, x, xh, t, w = _setup(4, n, ny, nx)
     w[:] = 1.0
@@ -82,6 +83,33 @@ def test_gradients_at_band_edges_match_oracle(n, ny, nx):
         sl = slice(l * cnn.PSZ, (l + 1) * cnn.PSZ)
         e = _rel(g[sl], rg[sl])
         _say(f"  {n}x{ny}x{nx} layer {l} gradient rel L2 {e:.2e}")
+        assert e < 5e-3, (l, e)
+
+
+def test_gradients_where_a_block_takes_several_bands(monkeypatch):
+    """516 bands on 512 blocks: the loss weighs 13 pixels alone, at the edges of the first and
+    last bands and of those that a block takes second (rows 1016 on of the second image).
+    Each single product of such a pixel, one tap of it, is more of its layer's gradient than
+    the tolerance, which the oracle's own terms show."""
+    n, ny, nx = 2, 1030, 16
+    net, p, x, xh, t, w = _setup(4, n, ny, nx)
+    w[:] = 0.0
+    for k, row in enumerate((0, 3, 4, ny - 1)):
+        w[0, row, 5 * k % nx] = 1.0
+    for k, row in enumerate((1015, 1016, 1019, 1020, 1023, 1024, 1027, 1028, 1029)):
+        w[1, row, 7 * k % nx] = 1.0
+    _, g = net.loss_grad(x, _dev(t), _dev(w), want_grad=True)
+    operands, product = [], cnn.conv_weight_grad
+    monkeypatch.setattr(cnn, "conv_weight_grad", lambda a, dz: (operands.append((a, dz)), product(a, dz))[1])
+    _, rg = cnn.loss_grad(p, xh, t, w, emulate=True)
+    for l, (a, dz) in zip(reversed(range(cnn.LAYERS)), operands):
+        sl = slice(l * cnn.PSZ, (l + 1) * cnn.PSZ)
+        norm = np.pad(np.linalg.norm(a, axis=-1), ((0, 0), (1, 1), (1, 1)))
+        terms = np.concatenate([norm[i, y:y + 3, c:c + 3].ravel() * np.linalg.norm(dz[i, y, c])
+                                for i, y, c in np.argwhere(w > 0)])
+        assert terms[terms > 0].min() > 5e-3 * np.linalg.norm(rg[sl])
+        e = _rel(g[sl], rg[sl])
+        _say(f"  layer {l} gradient rel L2 {e:.2e}, smallest term {terms[terms > 0].min() / np.linalg.norm(rg[sl]):.2e}")
         assert e < 5e-3, (l, e)
 
 
