@@ -636,16 +636,7 @@ template <int S, class T, class U> __device__ __forceinline__ void loadTensor(co
         c[s] = f[(2 * S + s) * ne + e];
     }
 }
-// The same with scalar field bases and the element's 32-bit byte offset (ldAt).
-template <int S, class T> __device__ __forceinline__ void loadTensorAt(const T* f, size_t ne, uint32_t off, T* a, T* b, T* c)
-{
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-        a[s] = ldAt(f + (0 * S + s) * ne, off);
-        b[s] = ldAt(f + (1 * S + s) * ne, off);
-        c[s] = ldAt(f + (2 * S + s) * ne, off);
-    }
-}
+// Stores with scalar field bases and the element's 32-bit byte offset (fieldAt).
 template <int S, class T> __device__ __forceinline__ void storeTensorAt(T* f, size_t ne, uint32_t off, const T* a, const T* b, const T* c)
 {
 #pragma unroll

@@ -31,13 +31,11 @@ struct TrArgs {
     const double* nvX;
     const double* nvY;
     const double* ops;
-    size_t opStride;
     double dt;
     int mode;
     const double* base; // the field the step starts from (RK2 and RK3 stages)
     double* out;
     double* raw;        // un-finished increment (periodic path)
-    bool withDirichlet;
     double* tally;      // per-element Dirichlet outflow accumulator (mass budget), or null
     double tallyW;      // weight of this stage's outflow in the step (1/R folded in on the sphere)
     Limits lim;         // limiters applied to the stage's result
@@ -989,7 +987,6 @@ template <int DG> struct TransportImpl final : TransportBase {
         a.nvX = nvX.p;
         a.nvY = nvY.p;
         a.ops = ops.p;
-        a.opStride = mesh.uniform ? 1 : mesh.ne;
         a.dt = dt;
         return a;
     }
