@@ -1583,10 +1583,11 @@ __device__ __forceinline__ void momentumFrozen(const NodeArgs& a, const NodeFz& 
 template <int CG> using FusedTile = TileShape<CG, 31, 7>;
 static_assert(FusedTile<2>::HX * FusedTile<2>::HY == kBlock, "fused tile must give one element per thread");
 
-// Node update policies of nodeTileUpdate: In is what a node loads before its update;
-// kAllNodes runs the update on Dirichlet nodes too (their divergence is zero, their
-// velocity is zeroed after the update).
-// mEVP (VPCGDynamicsKernel.hpp:132-172) from the frozen coefficients; Dirichlet nodes skip it.
+// Node update policies of nodeTileUpdate: In is what a node loads before its update. The
+// update runs on every node, and the velocity of a Dirichlet node is zeroed after it;
+// kAllNodes: the update writes more than that velocity, so that a Dirichlet node's
+// divergence must be zero in it.
+// mEVP (VPCGDynamicsKernel.hpp:132-172) from the frozen coefficients.
 struct MevpNode {
     using In = NodeFz;
     static constexpr bool kAllNodes = false;
@@ -1921,9 +1922,10 @@ template <int CG, int DG> __global__ __launch_bounds__(kBlock) void k_residual_f
 // k_mevp_fused, in the same order, from the same operands (a halo value identically in
 // every tile that computes it); the compiler may still fuse a multiply-add differently
 // in the two kernels, which moves a value by an ulp.
-// FP64: 13 x 13 owned elements on 256 threads. FP32, bound by instruction issue and with
-// half the LDS per value: 29 x 13 on 512 threads, 2.47 element updates per owned element and
-// two subcycles instead of 2.67.
+// FP64: 13 x 13 owned elements on 256 threads. FP32, which issues more
+// instructions for its rounding (VALU 68% busy at 1024 x 1024, FP64 50%) and needs half the
+// LDS per value: 29 x 13 on 512 threads, 2.47 element updates per owned element and two
+// subcycles instead of 2.67.
 // FP64 is bound by how much of its memory traffic overlaps its arithmetic: a block alone
 // issues for 8 us and took 18. Every wait for a load covers the loads issued before it
 // (they return in order), so the block issues them in the order of their use, well ahead:
@@ -2510,8 +2512,8 @@ __device__ __forceinline__ void divergenceGeomFrom(const double* geo, size_t ne,
 // Bound by its traffic, near the copy rate on large meshes, and by the latency of one block
 // on small ones: nothing of an inverse mass is streamed (the projection goes through the
 // Gauss weights), the latitudes stay in LDS from the strain to the divergence, and all that
-// the element reads is issued before the strain (182 VGPRs, two blocks per CU; three blocks
-// of 168 that load strength and stress where they are used: 59.0 and 12.9 us in place of
+// the element reads is issued before the strain (204 VGPRs on the sphere, 170 on a plane, two
+// blocks per CU; three blocks of 168 that load strength and stress where they are used: 59.0 and 12.9 us in place of
 // the last figures). Per subcycle, in these steps: 512 x 512 spherical patch 86.6 -> 64.4 ->
 // 61.9 (sum factorisations) -> 58.2 us, 154 x 121 16.5 -> 13.4 -> 12.5 us. Loading the
 // first nodes' terms before the divergence as well was slower (60.0 us).
@@ -3068,16 +3070,6 @@ __device__ __forceinline__ constexpr int basisFX(int k) { return k == 1 || k == 
 __device__ __forceinline__ constexpr int basisGY(int k) { return k == 2 || k == 5 || k == 6 ? 1 : (k == 4 || k == 7 ? 2 : 0); }
 __device__ __forceinline__ constexpr double legendre01(int i, double t) { return i == 0 ? 1.0 : (i == 1 ? t : t * t - 1.0 / 12.0); }
 
-// bbmElement for the one-pass kernel on an affine uniform mesh, with the operators of
-// elementAffineCompute: the Gauss-point strain is the exact gradient of the CG velocity by
-// sum factorisation (ocean elements; land elements interpolate their stored strain), both
-// projections are psi_k(q) w_q / m_k literals, and every DG field is evaluated per Gauss
-// row from its three row coefficients. The strain is not stored.
-// The caller's per-thread column gp(r), r = 4 q + {0, 1, 2, 3} for Gauss point q, holds
-// first the previous stress and damage interpolated there (a pre-pass, one field at a
-// time), then the new ones; the projection runs after the Gauss loop in the order q. So
-// neither the previous coefficients nor the 30 projection sums are live while the point
-// arithmetic runs. Ocean and land elements take separate Gauss loops.
 // What the brittle update of an element reads besides its velocities: loaded at once, ahead
 // of the strain, so that one wait covers it (the loads return while the strain is formed).
 template <int CG, int DG> struct BrittleState {
@@ -3141,6 +3133,15 @@ __device__ __forceinline__ void bbmGaussLoop(const BrittleArgs& b, const double*
         }
     }
 }
+// bbmElement for the one-pass kernel on an affine uniform mesh, with the operators of
+// elementAffineCompute: the Gauss-point strain is the exact gradient of the CG velocity by
+// sum factorisation (land elements take their stored strain there), both projections are
+// the fixed sums of projectionMoments, and every DG field is evaluated through its row
+// coefficients. The strain is not stored.
+// The caller's per-thread column gp(r), r = 4 q + {0, 1, 2, 3} for Gauss point q, holds
+// first the previous stress and damage interpolated there, then the new ones, which are
+// projected after the point loop: neither the previous coefficients nor the projection's
+// sums are live while the point arithmetic runs.
 template <int CG, int DG, bool POW5, class GP>
 __device__ __forceinline__ void bbmElementAffine(const ElemArgs& a, const BrittleArgs& b, int e, double* acc1,
     double* acc2, double* acc3, double* accD, GP&& gp)
@@ -3299,7 +3300,8 @@ struct BrittleFusedArgs {
     double* vOut;
     const double* geo; // GeoLayout tables of a general mesh (k_bbm_fused_geom)
 };
-// Bound by instruction issue and by the latency of its loads at two blocks per CU. 512 x 512:
+// Bound by latency at two blocks per CU: the VALU is 33% busy, a wave issues in 30% of its time,
+// waits for memory in 30% and for an instruction to issue in 40%. 512 x 512:
 // 78.7 -> 71.7 us per substep (sum factorisations, one point loop for ocean and land, short
 // roots) -> 66.5 (all loads ahead of the strain; the two quotients of a point computed
 // before the conditions that select them, so that the points' chains overlap). Loading the
@@ -4153,9 +4155,11 @@ template <int CG, int DG> struct DynImpl final : DynBase {
         checkLaunch("strain");
     }
     // Two subcycles per pass: uniform meshes without periodic segments (FP64 or FP32), by default
-    // from NSDG_PAIR_MIN_ELEMENTS up (every such mesh: faster per step than k_mevp_fused
-    // from 128^2 to 2048^2 except near 320^2, within 3.5% there)
-    // (below, the state largely stays in the memory-side cache).
+    // from NSDG_PAIR_MIN_ELEMENTS up (every such mesh). 100 subcycles with pairs against single
+    // passes, CG2 in FP64: 64^2 0.63 against 1.27 ms, 272^2 1.10 against 1.57, 288^2 (513 tiles,
+    // one more than are resident) 1.44 against 1.58, 320^2 1.49 against 1.70, 352^2 1.96 against
+    // 2.11, 384^2 1.93 against 2.24, 512^2 3.12 against 3.85; CG1 0.55 to 0.84 of the single
+    // passes from 64^2 to 512^2. FP32: 0.70 to 0.98 from 128^2 to 1024^2, 1.06 at 320^2 alone.
     bool pairSubcycles() const
     {
         const bool can = fusedSubcycle() && mesh.uniform;

@@ -352,7 +352,6 @@ class BBMDynamicsKernel(MEVPDynamicsKernel):
     dt / nSteps (BrittleCGDynamicsKernel.hpp:92-134). The extra DG field "damage" is set
     and read like hice; the averaged velocity is the CG vector "avgU" / "avgV". The
     mEVP-only facilities (momentum residual, FP32 variant, learned warm start) raise.
-    Uniform meshes only.
     """
 
     def __init__(self, cg_degree=2, dg_adv=6, params=None, meb=None, **overrides):
