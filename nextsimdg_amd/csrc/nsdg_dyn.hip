@@ -2513,10 +2513,11 @@ __device__ __forceinline__ void divergenceGeomFrom(const double* geo, size_t ne,
 // on small ones: nothing of an inverse mass is streamed (the projection goes through the
 // Gauss weights), the latitudes stay in LDS from the strain to the divergence, and all that
 // the element reads is issued before the strain (204 VGPRs on the sphere, 170 on a plane, two
-// blocks per CU; three blocks of 168 that load strength and stress where they are used: 59.0 and 12.9 us in place of
-// the last figures). Per subcycle, in these steps: 512 x 512 spherical patch 86.6 -> 64.4 ->
-// 61.9 (sum factorisations) -> 58.2 us, 154 x 121 16.5 -> 13.4 -> 12.5 us. Loading the
-// first nodes' terms before the divergence as well was slower (60.0 us).
+// blocks per CU; three blocks of 168 that load strength and stress where they are used:
+// 59.0 and 12.9 us in place of the last figures). Per subcycle, in these steps: 512 x 512
+// spherical patch 86.6 -> 64.4 -> 61.9 (sum factorisations) -> 58.2 us, 154 x 121 16.5 -> 13.4
+// -> 12.5 us. Loading the first nodes' terms before the divergence as well was slower (60.0
+// us).
 template <int CG, int DG, bool SPH>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_mevp_fused_geom(FusedArgs f)
 {
@@ -4156,8 +4157,8 @@ template <int CG, int DG> struct DynImpl final : DynBase {
     }
     // Two subcycles per pass: uniform meshes without periodic segments (FP64 or FP32), by default
     // from NSDG_PAIR_MIN_ELEMENTS up (every such mesh). 100 subcycles with pairs against single
-    // passes, CG2 in FP64: 64^2 0.63 against 1.27 ms, 272^2 1.10 against 1.57, 288^2 (513 tiles,
-    // one more than are resident) 1.44 against 1.58, 320^2 1.49 against 1.70, 352^2 1.96 against
+    // passes, CG2 in FP64: 64^2 0.63 against 1.27 ms, 272^2 1.10 against 1.57, 288^2 (529 tiles,
+    // 512 are resident) 1.44 against 1.58, 320^2 1.49 against 1.70, 352^2 1.96 against
     // 2.11, 384^2 1.93 against 2.24, 512^2 3.12 against 3.85; CG1 0.55 to 0.84 of the single
     // passes from 64^2 to 512^2. FP32: 0.70 to 0.98 from 128^2 to 1024^2, 1.06 at 320^2 alone.
     bool pairSubcycles() const
