@@ -3302,7 +3302,7 @@ struct BrittleFusedArgs {
     const double* geo; // GeoLayout tables of a general mesh (k_bbm_fused_geom)
 };
 // Bound by latency at two blocks per CU: the VALU is 33% busy, a wave issues in 30% of its time,
-// waits for memory in 30% and for an instruction to issue in 40%. 512 x 512:
+// is at a wait (memory, LDS, the block) in 30% and waits to issue in 40%. 512 x 512:
 // 78.7 -> 71.7 us per substep (sum factorisations, one point loop for ocean and land, short
 // roots) -> 66.5 (all loads ahead of the strain; the two quotients of a point computed
 // before the conditions that select them, so that the points' chains overlap). Loading the
