@@ -186,7 +186,7 @@ def brittle_leg(nx, steps, warmup, dt=120.0, seed=0, traffic_path=None, warp=0.0
     k.set_profiling(True)
     run_steps(k, off, L, warmup + steps, 1, dt)
     k.synchronize()
-    names = ("bbm_fused", "strain", "transport_op", "limit", "dg2cg", "cg2dg", "ssh_gradient")
+    names = ("bbm_fused", "strain", "transport_op", "dg2cg", "cg2dg", "ssh_gradient")
     stats = {n: k.kernel_stats(n) for n in names}
     k.set_profiling(False)
     c, tot = stats["bbm_fused"]
