@@ -767,7 +767,7 @@ void HostIO::toHost(void* hostp, const void* src, size_t bytes, hipStream_t s)
         NSDG_HIP(hipStreamSynchronize(s));
         return;
     }
-    const int n = static_cast<int>(std::min<size_t>(kThreads, bytes / kMinShare));
+    const int n = std::clamp(static_cast<int>(bytes / kShare), 2, kThreads);
     reserve(n);
     const size_t share = ((bytes + n - 1) / n + 4095) & ~size_t(4095);
     int device = 0;

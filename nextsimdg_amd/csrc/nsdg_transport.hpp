@@ -40,14 +40,15 @@ struct TransportBase {
 // split, into fresh pages (whose faults the threads share): 8 MiB 2.2 -> 1.2 to 1.5 ms, 32 MiB
 // 8.9 -> 5.4; into pages in use: 4 MiB 0.23 -> 0.24, 8 MiB 0.47 -> 0.44, 32 MiB 1.8 -> 1.6; the
 // first copy of a handle, which pins its slots, into pages in use: 4 MiB 0.27 -> 0.32, 8 MiB
-// 0.53 -> 0.54, 16 MiB 1.02 -> 0.93. Below 8 MiB a copy stays with the runtime; a thread
-// takes at least 4 MiB, so that a copy pays for its slots; eight threads copied no faster
-// than four and took twice as long to pin theirs. Slots of 256 KiB: 32 MiB 2.4 ms.
+// 0.53 -> 0.54, 16 MiB 1.02 -> 0.93. Below 6 MiB a copy stays with the runtime; two threads take
+// it up to 24 MiB and one more for each 8 MiB beyond, so that a copy pays for its slots; eight
+// threads copied no faster than four and took twice as long to pin theirs. Slots of 256 KiB:
+// 32 MiB 2.4 ms.
 // Page-locked and device destinations stay with the runtime (2048 x 2048 cell means 0.6 ms),
 // and so do uploads: it reads pageable memory faster (preparing the 512 x 512 box took 15
 // ms through the slots, 11 without).
 struct HostIO {
-    static constexpr size_t kMinSplit = size_t(1) << 23, kSlot = size_t(1) << 19, kMinShare = 8 * kSlot;
+    static constexpr size_t kMinSplit = size_t(6) << 20, kSlot = size_t(1) << 19, kShare = size_t(1) << 23;
     static constexpr int kThreads = 4;
     DBuf<double> scratch;
     HostIO() = default;

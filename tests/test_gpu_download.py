@@ -59,9 +59,9 @@ def _round_trip(k, name, ncomp, scale):
     assert np.array_equal(out, want), (name, ncomp, np.flatnonzero(out != want)[:4])
 
 
-# 2^20 values are 8 MiB, from where a copy is split: one value less, that size, a row more,
-# odd sizes; 513 x 515 with 8 components gives four threads 8 slots each and a remainder.
-@pytest.mark.parametrize("nx,ny", [(1025, 1023), (1024, 1024), (1024, 1025), (1033, 1021), (513, 515), (397, 263)])
+# 3 * 2^18 values are 6 MiB, from where a copy is split: that size, two values less, a row
+# more, odd sizes; with 8 components four threads, 513 x 515 two of 16 slots and a remainder.
+@pytest.mark.parametrize("nx,ny", [(1024, 768), (393215, 2), (1024, 769), (1033, 1021), (513, 515), (397, 263)])
 def test_fields_round_trip_around_the_split(nx, ny):
     print(f"round trip {nx}x{ny}", flush=True)
     k = _kernel(nx, ny)
@@ -75,7 +75,7 @@ def test_fields_round_trip_around_the_split(nx, ny):
 
 
 def test_one_handle_small_large_small():
-    """Plain, two threads, four (new slots), two again, plain; other values each time."""
+    """Two threads, four (new slots), two again, with other values each time; then plain copies."""
     k = _kernel(1061, 997)
     for i, (name, ncomp) in enumerate([("ssh", 1), ("s11", 1), ("s11", 8), ("s22", 1), ("hice", 6), ("s11", 1)]):
         _round_trip(k, name, ncomp, 1.0 + i)
