@@ -3880,7 +3880,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
         need();
         double* c = cgRef(n);
         require(c != nullptr, "unknown CG vector " + n);
-        io.toHost(out, c, nn * sizeof(double), s);
+        io.toHost(out, c, nn, s);
     }
     void setCG(const std::string& n, const double* in) override
     {
@@ -4827,7 +4827,7 @@ template <int CG, int DG> struct DynImpl final : DynBase {
         std::memcpy(buf.data(), &hd, sizeof hd);
         size_t off = sizeof(Header);
         for (auto& pr : stateParts()) {
-            io.toHost(buf.data() + off, pr.first, pr.second * sizeof(double), s);
+            io.toHost(reinterpret_cast<double*>(buf.data() + off), pr.first, pr.second, s);
             off += pr.second * sizeof(double);
         }
         NSDG_HIP(hipStreamSynchronize(s));

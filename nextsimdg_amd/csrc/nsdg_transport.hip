@@ -710,6 +710,14 @@ __global__ void k_fill(double* p, size_t n, double v)
         p[t] = v;
 }
 
+// The contents of one pinned slot (n values), stored into host memory by the kernel itself;
+// 16-byte accesses where the source allows them (a field's components start at any value).
+template <class T> __global__ __launch_bounds__(kBlock) void k_to_slot(T* dst, const T* src, size_t n)
+{
+    const size_t t = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (t < n)
+        dst[t] = src[t];
+}
 HostIO::~HostIO() { release(); }
 void HostIO::release()
 {
@@ -728,37 +736,43 @@ void HostIO::reserve(int n)
     if (n <= threads)
         return;
     release();
-    NSDG_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), 2 * n * kSlot, hipHostMallocDefault));
+    NSDG_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), 2 * n * kSlot * sizeof(double), hipHostMallocCoherent));
     for (int i = 0; i < 2 * n; ++i)
         NSDG_HIP(hipEventCreateWithFlags(&done[i], hipEventDisableTiming));
     threads = n;
 }
 // One thread's share of a copy, slot by slot through its two pinned slots.
-void HostIO::part(char* host, const char* dev, size_t bytes, int t, hipStream_t s)
+void HostIO::part(double* host, const double* dev, size_t values, int t, hipStream_t s)
 {
-    const size_t n = (bytes + kSlot - 1) / kSlot;
-    const auto size = [&](size_t i) { return std::min(kSlot, bytes - i * kSlot); };
+    const size_t n = (values + kSlot - 1) / kSlot;
+    const auto size = [&](size_t i) { return std::min(kSlot, values - i * kSlot); };
     const auto slot = [&](size_t i) { return pinned + (2 * t + (i & 1)) * kSlot; };
     const auto issue = [&](size_t i) {
-        NSDG_HIP(hipMemcpyAsync(slot(i), dev + i * kSlot, size(i), hipMemcpyDeviceToHost, s));
+        const double* const from = dev + i * kSlot;
+        const size_t m = size(i);
+        if ((reinterpret_cast<uintptr_t>(from) & 15u) == 0 && m % 2 == 0)
+            k_to_slot<<<blocksFor(m / 2), kBlock, 0, s>>>(
+                reinterpret_cast<double2*>(slot(i)), reinterpret_cast<const double2*>(from), m / 2);
+        else
+            k_to_slot<<<blocksFor(m), kBlock, 0, s>>>(slot(i), from, m);
+        checkLaunch("to_slot");
         NSDG_HIP(hipEventRecord(done[2 * t + (i & 1)], s));
     };
     for (size_t i = 0; i < std::min<size_t>(2, n); ++i)
         issue(i);
     for (size_t i = 0; i < n; ++i) {
         NSDG_HIP(hipEventSynchronize(done[2 * t + (i & 1)]));
-        std::memcpy(host + i * kSlot, slot(i), size(i));
+        std::memcpy(host + i * kSlot, slot(i), size(i) * sizeof(double));
         if (i + 2 < n)
             issue(i + 2);
     }
 }
-void HostIO::toHost(void* hostp, const void* src, size_t bytes, hipStream_t s)
+void HostIO::toHost(double* host, const double* dev, size_t values, hipStream_t s)
 {
-    char* const host = static_cast<char*>(hostp);
-    const char* const dev = static_cast<const char*>(src);
+    const size_t bytes = values * sizeof(double);
     // page-locked or device memory of the caller's: the copy engine writes it itself
     hipPointerAttribute_t at {};
-    const bool known = bytes >= kMinSplit && hipPointerGetAttributes(&at, hostp) == hipSuccess
+    const bool known = bytes >= kMinSplit && hipPointerGetAttributes(&at, host) == hipSuccess
         && at.type != hipMemoryTypeUnregistered;
     (void)hipGetLastError(); // asking about ordinary memory is no error
     if (bytes < kMinSplit || known) {
@@ -767,15 +781,15 @@ void HostIO::toHost(void* hostp, const void* src, size_t bytes, hipStream_t s)
         NSDG_HIP(hipStreamSynchronize(s));
         return;
     }
-    const int n = std::clamp(static_cast<int>(bytes / kShare), 2, kThreads);
+    const int n = static_cast<int>(std::clamp<size_t>(bytes / kShare, 2, kThreads));
     reserve(n);
-    const size_t share = ((bytes + n - 1) / n + 4095) & ~size_t(4095);
+    const size_t share = ((values + n - 1) / n + 511) & ~size_t(511); // whole pages of an aligned field
     int device = 0;
     NSDG_HIP(hipGetDevice(&device));
     std::exception_ptr failed[kThreads];
     const auto run = [&](int t) noexcept {
         try {
-            const size_t lo = std::min(bytes, t * share), hi = std::min(bytes, lo + share);
+            const size_t lo = std::min(values, t * share), hi = std::min(values, lo + share);
             NSDG_HIP(hipSetDevice(device));
             if (hi > lo)
                 part(host + lo, dev + lo, hi - lo, t, s);
@@ -816,14 +830,14 @@ void uploadSoA(HostIO& io, const double* host, size_t n, int nc, double* dst, hi
 void downloadSoA(HostIO& io, const double* src, size_t n, int nc, double* host, hipStream_t s)
 {
     if (nc == 1) {
-        io.toHost(host, src, n * sizeof(double), s);
+        io.toHost(host, src, n, s);
         return;
     }
     if (io.scratch.n < n * nc)
         io.scratch.alloc(n * nc);
     k_soa_to_aos<<<blocksFor(n * nc), kBlock, 0, s>>>(src, n, nc, io.scratch.p);
     checkLaunch("soa_to_aos");
-    io.toHost(host, io.scratch.p, n * nc * sizeof(double), s);
+    io.toHost(host, io.scratch.p, n * nc, s);
 }
 void deviceFill(double* p, size_t n, double v, hipStream_t s)
 {

@@ -36,34 +36,37 @@ struct TransportBase {
 // of the layout conversion. Of one handle, so used by one thread at a time.
 // The runtime copies into pageable memory through its own staging, one chunk and one core
 // at a time. From kMinSplit bytes up the range is split over a few threads, each with two
-// pinned slots, one filled by the copy engine while a core empties the other. Plain against
-// split, into fresh pages (whose faults the threads share): 8 MiB 2.2 -> 1.2 to 1.5 ms, 32 MiB
-// 8.9 -> 5.4; into pages in use: 4 MiB 0.23 -> 0.24, 8 MiB 0.47 -> 0.44, 32 MiB 1.8 -> 1.6; the
-// first copy of a handle, which pins its slots, into pages in use: 4 MiB 0.27 -> 0.32, 8 MiB
-// 0.53 -> 0.54, 16 MiB 1.02 -> 0.93. Below 6 MiB a copy stays with the runtime; two threads take
-// it up to 24 MiB and one more for each 8 MiB beyond, so that a copy pays for its slots; eight
-// threads copied no faster than four and took twice as long to pin theirs. Slots of 256 KiB:
-// 32 MiB 2.4 ms.
+// pinned slots: a kernel stores into one while a core empties the other. (Copies into the
+// slots by the copy engine fell to 4.7 GB/s for hundreds of copies at a time in processes with
+// several handles: 67 MB in 14.3 ms, by the runtime 6.3, by the kernel 2.3.)
+// Plain against split, into fresh pages (whose faults the threads share): 8 MiB 2.2 -> 2.0 ms,
+// 16 MiB 4.5 -> 3.8, 32 MiB 8.9 -> 5.6; into pages in use: 8 MiB 0.47 -> 0.36, 32 MiB 1.85 -> 0.97;
+// the first copy of a handle, which pins its slots, into pages in use: 8 MiB 0.53 -> 0.46, 16
+// MiB 1.02 -> 0.67; a new transport handle with one step at 512 x 512 (13 MB) 5.24 -> 5.11. Below
+// 6 MiB a copy stays with the runtime (4 MiB 0.23 ms, through slots 0.24 to 0.26 and 0.32 the
+// first time); two threads take it up to 24 MiB and one more for each 8 MiB beyond, so that a
+// copy pays for its slots.
 // Page-locked and device destinations stay with the runtime (2048 x 2048 cell means 0.6 ms),
 // and so do uploads: it reads pageable memory faster (preparing the 512 x 512 box took 15
 // ms through the slots, 11 without).
 struct HostIO {
-    static constexpr size_t kMinSplit = size_t(6) << 20, kSlot = size_t(1) << 19, kShare = size_t(1) << 23;
+    static constexpr size_t kMinSplit = size_t(6) << 20, kShare = size_t(1) << 23; // bytes
+    static constexpr size_t kSlot = size_t(1) << 16;                            // values
     static constexpr int kThreads = 4;
     DBuf<double> scratch;
     HostIO() = default;
     HostIO(const HostIO&) = delete;
     HostIO& operator=(const HostIO&) = delete;
     ~HostIO();
-    void toHost(void* host, const void* src, size_t bytes, hipStream_t s);
+    void toHost(double* host, const double* dev, size_t values, hipStream_t s);
 
 private:
-    char* pinned = nullptr; // 2 slots per thread, for `threads` threads
+    double* pinned = nullptr; // 2 slots per thread, for `threads` threads
     int threads = 0;
     hipEvent_t done[2 * kThreads] = {};
     void reserve(int n);
     void release();
-    void part(char* host, const char* dev, size_t bytes, int t, hipStream_t s);
+    void part(double* host, const double* dev, size_t values, int t, hipStream_t s);
 };
 
 // Owning wrapper used by the C ABI (mesh + transport + stream).
